@@ -31,7 +31,8 @@ inline hipError_t ensure_lds_limit(const void *fn, int bytes) {
 // attribute while a stream is being captured into a graph.
 hipError_t chain_prepare_lds();
 hipError_t q6_prepare_lds();
-// The same for every instantiation of the prefill / grouped GEMM (gemm_f16.hip).
+// The same for every instantiation of the prefill / grouped GEMMs (gemm_f16.hip).
 hipError_t gemm_prepare_lds();
+hipError_t gemm_wide_prepare_lds();  // gemm_wide.hip
 
 }  // namespace rce_qmm

@@ -95,6 +95,10 @@ rce_qmm_status run_gemm(const void *a_dev, bool a_f16, size_t t_rows, const DevW
     }
     if (reinterpret_cast<uintptr_t>(a) % 16)
         return fail(RCE_QMM_BAD_SHAPE, "F16 activations of the F16_MFMA GEMM must be 16-byte aligned");
+    if (gemm_wide_preferred(dw, t_rows)) {  // large tiles, F16 weights
+        HIP_TRY(launch_gemm_wide(dw, a, t_rows, out_dev, s));
+        return RCE_QMM_OK;
+    }
     if (gemm_supports(dw.dtype, dw.n_cols) || gemm_q8_supports(dw.dtype, dw.n_cols)) {
         // The kernel's activation offsets are 32-bit: slices of whole
         // 128-row tiles below 2^32 bytes each (each output's sum does not
@@ -240,6 +244,7 @@ rce_qmm_status rce_qmm_context_create(int device, rce_qmm_context **out) {
     HIP_TRY(rce_qmm::chain_prepare_lds());
     HIP_TRY(rce_qmm::q6_prepare_lds());
     HIP_TRY(rce_qmm::gemm_prepare_lds());
+    HIP_TRY(rce_qmm::gemm_wide_prepare_lds());
     hipStream_t s = nullptr;
     HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     rce_qmm_context *c = new (std::nothrow) rce_qmm_context();

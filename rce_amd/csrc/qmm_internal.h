@@ -374,6 +374,12 @@ hipError_t launch_gemm_gen(const DevWeight &w, const void *a_f16, size_t M, floa
 // The tile rows the GEMM uses for M = rows_hint (plain) or for a mean of
 // rows_hint rows per expert (grouped).
 int gemm_tile_rows(size_t rows_hint, bool grouped);
+// The same in larger tiles (gemm_wide.hip) and for F16 weights: whether the
+// call is taken there, and its launch.
+bool gemm_wide_preferred(const DevWeight &w, size_t M);
+hipError_t launch_gemm_wide(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s);
+// Compute units of the current device (0 if unknown), read once per device.
+int cu_count();
 // f32 activations -> binary16 (round to nearest even) for the GEMM.
 hipError_t launch_f32_to_f16(const float *src, void *dst, size_t n, hipStream_t s);
 
