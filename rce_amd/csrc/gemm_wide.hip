@@ -211,13 +211,6 @@ struct WideTile {
     }
 };
 
-template <int N, int I = 0, class Fn>
-__device__ __forceinline__ void static_for(Fn &&f) {
-    if constexpr (I < N) {
-        f(ic<I>{});
-        static_for<N, I + 1>(f);
-    }
-}
 template <int N>
 __device__ __forceinline__ void wait_lgkm() {
     static_assert(N >= 0 && N < 16, "lgkmcnt range");

@@ -34,5 +34,6 @@ hipError_t q6_prepare_lds();
 // The same for every instantiation of the prefill / grouped GEMMs (gemm_f16.hip).
 hipError_t gemm_prepare_lds();
 hipError_t gemm_wide_prepare_lds();  // gemm_wide.hip
+hipError_t q8_mfma_prepare_lds();    // gemv_q8_mfma.hip
 
 }  // namespace rce_qmm

@@ -127,5 +127,14 @@ __device__ __forceinline__ half8 join8(half2v a, half2v b, half2v c, half2v d) {
 template <int U>
 using ic = std::integral_constant<int, U>;
 
+// f(ic<I>{}) for I = 0 .. N - 1.
+template <int N, int I = 0, class Fn>
+__device__ __forceinline__ void static_for(Fn &&f) {
+    if constexpr (I < N) {
+        f(ic<I>{});
+        static_for<N, I + 1>(f);
+    }
+}
+
 }  // namespace
 }  // namespace rce_qmm

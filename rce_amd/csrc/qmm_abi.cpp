@@ -140,13 +140,21 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     const bool widen = !mfma && a_dtype == T_F16;
     const bool preq = mode == RCE_QMM_MODE_Q8 && gemv_q8_pre_supports(dw.dtype, k, t_rows);
     const size_t f32_b = widen ? t_rows * k * sizeof(float) : 0;
-    const size_t q8_b = preq ? t_rows * (k + k / 8 + k / 4) : 0;  // xq, dx, s16
+    size_t q8_b = preq ? t_rows * (k + k / 8 + k / 4) : 0;  // xq, dx, s16
+    // Q8 on the int8 matrix cores: whole tiles of 16 tokens; where those do
+    // not fit the fixed scratch, the form that needs the documented bytes
+    bool mma = mode == RCE_QMM_MODE_Q8 && gemv_q8_mfma_supports(dw.dtype, k, t_rows) && gemv_q8_mfma_preferred(dw, t_rows);
+    if (mma) {
+        const size_t b = (t_rows + 15) / 16 * gemv_q8_tile_bytes(k);
+        if (fixed && align_up(f32_b, 256) + align_up(b, 256) > fixed_cap) mma = false;
+        else q8_b = b;
+    }
     const size_t f16_b = mfma && a_dtype == T_F32 ? t_rows * k * 2 : 0;
     BatchedScratch sc;
     rce_qmm_status st;
     if (fixed) {
         const size_t need = batched_scratch_bytes(dw, a_dtype, t_rows, mode);
-        if (need > fixed_cap)
+        if (!mma && need > fixed_cap)
             return fail(RCE_QMM_BAD_SHAPE, "the call needs " + std::to_string(need) + " bytes of scratch; the fixed scratch holds " +
                                                std::to_string(fixed_cap));
         unsigned char *p = static_cast<unsigned char *>(fixed);
@@ -172,6 +180,10 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     if (widen) {
         HIP_TRY(launch_f16_to_f32(static_cast<const uint16_t *>(a_dev), sc.a_f32, t_rows * k, s));
         a32 = sc.a_f32;
+    }
+    if (mma) {
+        HIP_TRY(launch_gemv_q8_mfma(dw, a32, t_rows, out_dev, sc.act_q, s));
+        return RCE_QMM_OK;
     }
     if (preq) {
         HIP_TRY(launch_gemv_q8_pre(dw, a32, t_rows, out_dev, sc.act_q, s));
@@ -245,6 +257,7 @@ rce_qmm_status rce_qmm_context_create(int device, rce_qmm_context **out) {
     HIP_TRY(rce_qmm::q6_prepare_lds());
     HIP_TRY(rce_qmm::gemm_prepare_lds());
     HIP_TRY(rce_qmm::gemm_wide_prepare_lds());
+    HIP_TRY(rce_qmm::q8_mfma_prepare_lds());
     hipStream_t s = nullptr;
     HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     rce_qmm_context *c = new (std::nothrow) rce_qmm_context();

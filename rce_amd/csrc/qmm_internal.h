@@ -309,16 +309,16 @@ hipError_t launch_gemv(const DevWeight &w, const float *a, size_t t_rows, float 
 hipError_t launch_gemv_q8_pre(const DevWeight &w, const float *a, size_t t_rows, float *out, void *ws,
                               hipStream_t s);
 bool gemv_q8_pre_supports(uint32_t dtype, size_t n_cols, size_t t_rows);
-// The int8 matrix-core form of the same (gemv_q8_mfma.hip): Q4_0 / Q8_0,
-// n_cols a multiple of 256, 2 or more tokens; preq as k_quantize_act writes
-// it (the ActLds layout of t_rows tokens).  Chosen where it is faster
-// (gemv_q8_mfma_preferred); RCE_QMM_Q8_MFMA=0 turns it off, =2 forces it
-// wherever it applies (same bits either way).
+// The int8 matrix-core form of the same (gemv_q8_mfma.hip): Q4_0, Q8_0, Q5_0,
+// Q4_1, Q4_K, Q5_K and Q6_K with n_cols a multiple of 256, 2 or more tokens,
+// in tiles of 16 tokens of gemv_q8_tile_bytes(n_cols) bytes of workspace
+// each.  Chosen where it is faster (gemv_q8_mfma_preferred);
+// RCE_QMM_Q8_MFMA=0 turns it off, =2 forces it wherever it applies (same
+// bits either way).
 bool gemv_q8_mfma_supports(uint32_t dtype, size_t n_cols, size_t t_rows);
-bool gemv_q8_mfma_preferred(size_t n_cols, size_t t_rows);
-bool gemv_q8_mfma_enabled();
-bool gemv_q8_mfma_forced();
-hipError_t launch_gemv_q8_mfma(const DevWeight &w, const unsigned char *preq, size_t t_rows, float *out, hipStream_t s);
+bool gemv_q8_mfma_preferred(const DevWeight &w, size_t t_rows);
+size_t gemv_q8_tile_bytes(size_t n_cols);
+hipError_t launch_gemv_q8_mfma(const DevWeight &w, const float *a, size_t t_rows, float *out, void *acts, hipStream_t s);
 GemvGeom pick_gemv_geom(const DevWeight &w, size_t t_rows, int mode);
 // Per-format launchers (gemv_<format>.hip), shape already chosen.
 hipError_t launch_gemv_q4_0(const DevWeight &w, const GemvGeom &g, const float *a, size_t t_rows, float *out,
@@ -452,6 +452,18 @@ enum GemmEpilogue { GEPI_F32 = 0, GEPI_SILU_F16 = 1, GEPI_SWIGLU_F16 = 2 };
 // dtype and shape shared by all experts; wtab is a device array of
 // DevWeight; a_rows: rows of A (bounds the loads); max_tiles bounds
 // n_tiles_dev[0].
+// The Q8 mode of grouped experts on the int8 matrix cores (gemv_q8_mfma.hip):
+// tiles of 16 slots.  launch_quantize_tiles fills `acts`
+// (gemv_q8_tile_bytes(k) per tile) from the rows of a: src Q8SRC_ROWS the
+// slots' tokens (tok_of_slot) or plain rows, Q8SRC_SILU silu(a[slot]),
+// Q8SRC_SWIGLU silu(a[slot]) * a2[slot]; launch_gemv_q8_grouped forms out[slot] =
+// wtab[expert] . acts (and out2 with wtab2, a second matrix of the same
+// shape).  At most 65535 tiles.
+enum : int { Q8SRC_ROWS = 0, Q8SRC_SILU = 1, Q8SRC_SWIGLU = 2 };
+hipError_t launch_quantize_tiles(int src, const float *a, const float *a2, size_t k, size_t t_rows, int n_tile_max,
+                                 const MoeTile *tiles, const int *n_tiles, const int *tok_of_slot, void *acts, hipStream_t s);
+hipError_t launch_gemv_q8_grouped(const DevWeight &w, const DevWeight *wtab, float *out, const DevWeight *wtab2, float *out2,
+                                  const void *acts, int n_tile_max, const MoeTile *tiles, const int *n_tiles, hipStream_t s);
 hipError_t launch_gemm_f16_grouped(const DevWeight &w, const DevWeight *wtab, const void *a_f16, size_t a_rows,
                                    const int *gather, const MoeTile *tiles, const int *n_tiles_dev, int max_tiles,
                                    int bm, int epi, void *out, const float *aux, hipStream_t s);
