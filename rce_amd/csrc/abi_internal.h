@@ -67,7 +67,11 @@ struct rce_qmm_context {
     rce_qmm_abi::Scratch act_q;  // several tokens' Q8 activations, quantized once per launch
     // grouped experts: grouping metadata, expert tables, stage buffers
     rce_qmm_abi::Scratch moe_meta, moe_wtab, moe_x, moe_h, moe_h16, moe_y, moe_u;
-    std::vector<rce_qmm::DevWeight> moe_wtab_host;  // what moe_wtab holds
+    std::vector<rce_qmm::DevWeight> moe_wtab_host;  // what moe_wtab holds (empty: unknown)
+    // EXACT / Q8 grouped calls: the grouping kernel's status word in mapped
+    // host memory, and the event after that kernel
+    int *moe_status = nullptr;
+    hipEvent_t moe_grouped = nullptr;
 };
 
 struct rce_qmm_weight {

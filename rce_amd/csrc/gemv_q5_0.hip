@@ -11,4 +11,8 @@ hipError_t launch_gemv_fx_q5_0(const FxLaunch &f, const GemvGeom &g, const float
     if (mode == 0) return launch_as_fx_nt<Q5_0Exact<1>, false>(f, g, a, s);
     return launch_as_fx_nt<Q5_0Q8<1>, true>(f, g, a, s);
 }
+hipError_t launch_gemv_grouped_q5_0(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s) {
+    if (mode == 0) return launch_as_grouped_tb<Q5_0Exact, false>(w, m, a, out, s);
+    return launch_as_grouped_tb<Q5_0Q8, true>(w, m, a, out, s);
+}
 }  // namespace rce_qmm

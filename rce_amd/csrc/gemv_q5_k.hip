@@ -11,4 +11,8 @@ hipError_t launch_gemv_fx_q5_k(const FxLaunch &f, const GemvGeom &g, const float
     if (mode == 0) return launch_as_fx_nt<Q5_KExact<1>, false>(f, g, a, s);
     return launch_as_fx_nt<Q5_KQ8<1>, true>(f, g, a, s);
 }
+hipError_t launch_gemv_grouped_q5_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s) {
+    if (mode == 0) return launch_as_grouped_tb<Q5_KExact, false>(w, m, a, out, s);
+    return launch_as_grouped_tb<Q5_KQ8, true>(w, m, a, out, s);
+}
 }  // namespace rce_qmm

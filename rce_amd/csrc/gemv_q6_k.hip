@@ -82,12 +82,25 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q6k(DevWeight w, const float
 // leave a chain (from +0.0, never -0.0) unchanged.
 constexpr int Q6_DS = 8;  // stages of loads a helper keeps in flight
 
+// GROUP (grouped experts): blockIdx.y is a tile of tiles[0 .. n_tiles[0]),
+// blockIdx.z the slot in it.
+template <bool GROUP>
 __global__ __launch_bounds__(256) void k_gemv_exact_q6k_split(DevWeight w, const float *__restrict__ A,
-                                                              float *__restrict__ out) {
+                                                              float *__restrict__ out, const DevWeight *__restrict__ wtab,
+                                                              const MoeTile *__restrict__ tiles,
+                                                              const int *__restrict__ n_tiles) {
     constexpr int SV = 96;  // chain steps per stage: 3 pairs
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const size_t t = blockIdx.y, row0 = (size_t)blockIdx.x * 64;
+    size_t t = blockIdx.y;
+    const size_t row0 = (size_t)blockIdx.x * 64;
+    if constexpr (GROUP) {
+        if ((int)blockIdx.y >= n_tiles[0]) return;
+        const MoeTile tl = tiles[blockIdx.y];
+        if ((int)blockIdx.z >= tl.rows) return;
+        w = wtab[tl.e];
+        t = (size_t)tl.r0 + blockIdx.z;
+    }
     const size_t k = w.n_cols;
     const int np = (int)(k / 256) * 8;  // pairs in a row
     const int ns = (np + 2) / 3;
@@ -189,20 +202,44 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q6k_split(DevWeight w, const
     }
 }
 
+size_t q6_split_lds(size_t k) { return (k + 4) * sizeof(float) + 2 * 96 * 64 * sizeof(float); }
+
 hipError_t launch_q6_split(const DevWeight &w, const float *a, size_t t_rows, float *out, hipStream_t s) {
-    const size_t lds = (w.n_cols + 4) * sizeof(float) + 2 * 96 * 64 * sizeof(float);
+    const size_t lds = q6_split_lds(w.n_cols);
     if (lds > 64 * 1024) {  // activations of a long row: more than the default 64 KB
-        const hipError_t e = ensure_lds_limit((const void *)k_gemv_exact_q6k_split, 160 * 1024);
+        const hipError_t e = ensure_lds_limit((const void *)k_gemv_exact_q6k_split<false>, 160 * 1024);
         if (e != hipSuccess) return e;
     }
     const dim3 grid((unsigned)((w.n_rows + 63) / 64), (unsigned)t_rows);
-    hipLaunchKernelGGL(k_gemv_exact_q6k_split, grid, dim3(256), lds, s, w, a, out);
+    hipLaunchKernelGGL(k_gemv_exact_q6k_split<false>, grid, dim3(256), lds, s, w, a, out, (const DevWeight *)nullptr,
+                       (const MoeTile *)nullptr, (const int *)nullptr);
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t q6_prepare_lds() { return ensure_lds_limit((const void *)k_gemv_exact_q6k_split, 160 * 1024); }
+hipError_t q6_prepare_lds() {
+    const hipError_t e = ensure_lds_limit((const void *)k_gemv_exact_q6k_split<false>, 160 * 1024);
+    return e != hipSuccess ? e : ensure_lds_limit((const void *)k_gemv_exact_q6k_split<true>, 160 * 1024);
+}
+
+hipError_t launch_gemv_grouped_q6_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s) {
+    if (mode != 0) return launch_as_grouped_tb<Q6_KQ8, true>(w, m, a, out, s);
+    if (w.n_cols > Q6_EXACT_LDS_K) return hipErrorInvalidValue;
+    const size_t lds = q6_split_lds(w.n_cols);
+    if (lds > 64 * 1024) {
+        const hipError_t e = ensure_lds_limit((const void *)k_gemv_exact_q6k_split<true>, 160 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    const dim3 grid((unsigned)((w.n_rows + 63) / 64), (unsigned)m.max_tiles, (unsigned)m.tb);
+    for (int i = 0; i < (m.wtab2 ? 2 : 1); i++) {
+        hipLaunchKernelGGL(k_gemv_exact_q6k_split<true>, grid, dim3(256), lds, s, w, static_cast<const float *>(a),
+                           i ? m.out2 : out, i ? m.wtab2 : m.wtab, m.tiles, m.n_tiles);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
 
 hipError_t launch_gemv_q6_k(const DevWeight &w, const GemvGeom &g, const float *a, size_t t_rows, float *out, int mode,
                             hipStream_t s) {

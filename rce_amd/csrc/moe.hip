@@ -165,16 +165,27 @@ __global__ __launch_bounds__(GT) void k_moe_prep(const int32_t *__restrict__ ids
                                                  int bm, int *__restrict__ offs, int *__restrict__ slot_of_pair,
                                                  int *__restrict__ tok_of_slot, MoeTile *__restrict__ tiles,
                                                  int *__restrict__ n_tiles, int *__restrict__ status,
+                                                 int *__restrict__ host_status, MoeBases bases,
                                                  const float *__restrict__ x, _Float16 *__restrict__ x16, size_t n_x) {
     __shared__ int cnt[GE_MAX * GT];
     __shared__ int wsum[GT / 64];
     if (blockIdx.x == 0) {
+        if (bases.tab)
+            for (int m = 0; m < bases.n_mat; m++)
+                if ((int)threadIdx.x < n_expert) {
+                    DevWeight dw = bases.proto[m];
+                    dw.base = bases.base[m * n_expert + threadIdx.x];
+                    bases.tab[m * n_expert + threadIdx.x] = dw;
+                }
         if (n_expert <= GE_MAX)
             group_by_expert_counts(ids, n_pairs, top_k, n_expert, bm, offs, slot_of_pair, tok_of_slot, tiles, n_tiles,
                                    status, cnt, wsum);
         else
             group_by_expert_scan(ids, n_pairs, top_k, n_expert, bm, offs, slot_of_pair, tok_of_slot, tiles, n_tiles,
                                  status, cnt);
+        // thread 0 wrote status[0]
+        if (host_status && threadIdx.x == 0)
+            __hip_atomic_store(host_status, status[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         return;
     }
     const size_t stride = (size_t)(gridDim.x - 1) * GT;
@@ -260,11 +271,14 @@ unsigned grid_1d(size_t n, unsigned bs) {
 
 hipError_t launch_moe_group(const int32_t *ids, size_t n_pairs, int top_k, int n_expert, int bm, int *offs,
                             int *slot_of_pair, int *tok_of_slot, MoeTile *tiles, int *n_tiles, int *status,
-                            const float *x, void *x16, size_t n_x, hipStream_t s) {
+                            int *host_status, const MoeBases &bases, const float *x, void *x16, size_t n_x,
+                            hipStream_t s) {
+    static_assert(sizeof(MoeBases) + 256 < 4096 && MOE_ARG_EXPERTS <= GT, "kernel argument space; a thread per expert");
     const unsigned conv = x16 && n_x ? grid_1d(n_x, GT) : 0;
     const unsigned blocks = 1 + (conv < 1024 ? conv : 1024);
     hipLaunchKernelGGL(k_moe_prep, dim3(blocks), dim3(GT), 0, s, ids, (int)n_pairs, top_k, n_expert, bm, offs,
-                       slot_of_pair, tok_of_slot, tiles, n_tiles, status, x, static_cast<_Float16 *>(x16), n_x);
+                       slot_of_pair, tok_of_slot, tiles, n_tiles, status, host_status, bases, x, static_cast<_Float16 *>(x16),
+                       n_x);
     return hipGetLastError();
 }
 

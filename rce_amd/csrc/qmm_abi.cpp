@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <new>
@@ -284,6 +285,8 @@ void rce_qmm_abi::context_release(rce_qmm_context *ctx) {
     for (Scratch *s : {&ctx->a_in, &ctx->a_f32, &ctx->out, &ctx->a_f16, &ctx->act_q, &ctx->moe_meta, &ctx->moe_wtab, &ctx->moe_x,
                        &ctx->moe_h, &ctx->moe_h16, &ctx->moe_y, &ctx->moe_u})
         if (s->p) (void)hipFree(s->p);
+    if (ctx->moe_grouped) (void)hipEventDestroy(ctx->moe_grouped);
+    if (ctx->moe_status) (void)hipHostFree(ctx->moe_status);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -489,6 +492,18 @@ rce_qmm_status rce_qmm_moe_router(const float *logits, size_t n_tokens, size_t n
 
 namespace {
 
+// Q8 grouped experts: the int8 matrix cores (tiles of 16 slots, whatever they
+// hold) against the decode kernels over tiles of two slots.  Measured (us,
+// decode / matrix cores, 8 experts top-2): Q4_K / Q6_K 2048x5632 at 1.5, 3 and
+// 6 rows per expert 86 / 106, 125 / 104, 169 / 109; Q4_0 4096x14336 at 3, 4 and
+// 6 161 / 189, 208 / 205, 277 / 209.
+bool moe_q8_mfma_preferred(double rows_per_expert, bool q6, bool by_tile) {
+    const char *e = std::getenv("RCE_QMM_Q8_MFMA");
+    const int mode = e ? std::atoi(e) : 1;
+    if (mode != 1) return mode == 2;
+    return !by_tile || rows_per_expert >= (q6 ? 2.5 : 4.0);
+}
+
 // The grouped experts: h = silu(W1 x) (w3 == nullptr, the benchmark's
 // two-matrix expert) or h = silu(W1 x) * (W3 x) (SwiGLU: W1 = gate, W3 =
 // up), y = W2 h, out = the decision-order combine.
@@ -543,10 +558,26 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
     // 1. stable grouping of the (token, decision) pairs by expert
     const size_t n_pairs = t_rows * top_k;
     if (n_pairs >= (size_t)1 << 30) return fail(RCE_QMM_BAD_SHAPE, "too many (token, decision) pairs");
-    // tile rows of the grouped GEMM for the average rows per expert (the
+    // EXACT and Q8: Q8 with several rows per expert on the int8 matrix cores
+    // (tiles of 16 slots), else the decode kernels over tiles of one or two
+    // slots; formats and sizes outside both, expert by expert.
+    const double per_expert = (double)n_pairs / (double)n_expert;
+    enum { BY_EXPERT, BY_TILE, Q8_MFMA } form = BY_EXPERT;
+    if (mode == RCE_QMM_MODE_EXACT || mode == RCE_QMM_MODE_Q8) {
+        const bool args = n_expert <= MOE_ARG_EXPERTS && n_pairs + n_expert <= 65535;
+        if (args && gemv_grouped_supports(a1.dtype, d_model, (int)mode) && gemv_grouped_supports(a2.dtype, d_ff, (int)mode))
+            form = BY_TILE;
+        if (args && mode == RCE_QMM_MODE_Q8 && gemv_q8_mfma_supports(a1.dtype, d_model, 2) &&
+            gemv_q8_mfma_supports(a2.dtype, d_ff, 2) && moe_q8_mfma_preferred(per_expert, a1.dtype == T_Q6_K || a2.dtype == T_Q6_K, form != BY_EXPERT))
+            form = Q8_MFMA;
+    }
+    // tile rows: for the average rows per expert in the grouped GEMM (the
     // generic kernel takes any tile of at most 128 rows; Q8_0 / Q6_K on the
     // nibble kernel only 128)
-    const int bm = (nib1 || nib2) && !q8n1 && !q8n2 ? gemm_tile_rows((n_pairs + n_expert - 1) / n_expert, true) : 128;
+    const int bm = form == Q8_MFMA ? 16
+                   : form == BY_TILE ? (per_expert > 1.0 ? 2 : 1)
+                   : (nib1 || nib2) && !q8n1 && !q8n2 ? gemm_tile_rows((n_pairs + n_expert - 1) / n_expert, true)
+                                                      : 128;
     const int max_tiles = (int)(n_pairs / bm + n_expert);
     const size_t meta_ints = (n_expert + 1) + 2 * n_pairs + 2;
     const size_t meta_bytes = align_up(meta_ints * 4, 16) + (size_t)max_tiles * sizeof(MoeTile);
@@ -562,31 +593,45 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
     if ((st = ensure(ctx, ctx->moe_y, n_pairs * d_model * sizeof(float), s))) return st;
     float *y = static_cast<float *>(ctx->moe_y.p);
 
+    // 2. expert tables: written by the grouping kernel from its arguments, or
+    // (many experts) uploaded when the expert set changes
+    const int n_mat = w3 ? 3 : 2;
+    const size_t tab_bytes = (size_t)n_mat * n_expert * sizeof(DevWeight);
+    MoeBases bases{};
+    if (mode == RCE_QMM_MODE_F16_MFMA || form != BY_EXPERT) {
+        const rce_qmm_weight *const *mats[3] = {w1, w2, w3};
+        if ((st = ensure(ctx, ctx->moe_wtab, tab_bytes, s))) return st;
+        if (n_expert <= MOE_ARG_EXPERTS) {
+            bases.tab = static_cast<DevWeight *>(ctx->moe_wtab.p);
+            bases.n_mat = n_mat;
+            for (int m = 0; m < n_mat; m++) {
+                bases.proto[m] = mats[m][0]->dw;
+                for (size_t e = 0; e < n_expert; e++) bases.base[m * n_expert + e] = mats[m][e]->dw.base;
+            }
+            ctx->moe_wtab_host.clear();
+        } else {
+            std::vector<DevWeight> tab((size_t)n_mat * n_expert);
+            for (int m = 0; m < n_mat; m++)
+                for (size_t e = 0; e < n_expert; e++) tab[m * n_expert + e] = mats[m][e]->dw;
+            if (ctx->moe_wtab_host.size() != tab.size() ||
+                std::memcmp(ctx->moe_wtab_host.data(), tab.data(), tab_bytes) != 0) {
+                HIP_TRY(hipStreamSynchronize(s));  // no kernel still reads the old table
+                HIP_TRY(hipMemcpy(ctx->moe_wtab.p, tab.data(), tab_bytes, hipMemcpyHostToDevice));
+                ctx->moe_wtab_host = tab;
+            }
+        }
+    }
+    const DevWeight *wtab1 = static_cast<const DevWeight *>(ctx->moe_wtab.p), *wtab2 = wtab1 + n_expert;
+    const DevWeight *wtab3 = wtab1 + 2 * n_expert;
+
     if (mode == RCE_QMM_MODE_F16_MFMA) {
-        // 2. expert tables (uploaded when the expert set changes)
-        std::vector<DevWeight> tab((w3 ? 3 : 2) * n_expert);
-        for (size_t e = 0; e < n_expert; e++) {
-            tab[e] = w1[e]->dw;
-            tab[n_expert + e] = w2[e]->dw;
-            if (w3) tab[2 * n_expert + e] = w3[e]->dw;
-        }
-        const size_t tab_bytes = tab.size() * sizeof(DevWeight);
-        if (ctx->moe_wtab_host.size() != tab.size() ||
-            std::memcmp(ctx->moe_wtab_host.data(), tab.data(), tab_bytes) != 0) {
-            if ((st = ensure(ctx, ctx->moe_wtab, tab_bytes, s))) return st;
-            HIP_TRY(hipStreamSynchronize(s));  // no kernel still reads the old table
-            HIP_TRY(hipMemcpy(ctx->moe_wtab.p, tab.data(), tab_bytes, hipMemcpyHostToDevice));
-            ctx->moe_wtab_host = tab;
-        }
-        const DevWeight *wtab1 = static_cast<const DevWeight *>(ctx->moe_wtab.p), *wtab2 = wtab1 + n_expert;
-        const DevWeight *wtab3 = wtab1 + 2 * n_expert;
         // 3. the grouping, and x -> f16 in the same launch; W1 GEMM on the
         // rows gathered per slot, storing f16 silu(W1 x) (SwiGLU: the gate
         // products in f32, then the up GEMM stores f16 silu(g) * u)
         if ((st = ensure(ctx, ctx->moe_x, t_rows * d_model * 2, s))) return st;
         if ((st = ensure(ctx, ctx->moe_h16, n_pairs * d_ff * 2, s))) return st;
         HIP_TRY(launch_moe_group(ids_dev, n_pairs, (int)top_k, (int)n_expert, bm, offs, slot_of_pair, tok_of_slot,
-                                 tiles, n_tiles, status, x_dev, ctx->moe_x.p, t_rows * d_model, s));
+                                 tiles, n_tiles, status, nullptr, bases, x_dev, ctx->moe_x.p, t_rows * d_model, s));
         auto grouped = [&](bool nibble, const DevWeight &w, const DevWeight *wtab, const void *a, size_t a_rows,
                            const int *gather, int epi, void *out, const float *aux) {
             return nibble
@@ -604,10 +649,64 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
         }
         // 4. W2 GEMM on the slots themselves
         HIP_TRY(grouped(nib2 || q8n2, a2, wtab2, ctx->moe_h16.p, n_pairs, nullptr, GEPI_F32, y, nullptr));
+    } else if (form != BY_EXPERT) {
+        // The grouping's status comes back through mapped host memory: the
+        // host waits for that kernel only, with the products already queued.
+        if (!ctx->moe_status)
+            HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&ctx->moe_status), sizeof(int), hipHostMallocDefault));
+        if (!ctx->moe_grouped) HIP_TRY(hipEventCreateWithFlags(&ctx->moe_grouped, hipEventDisableTiming));
+        if ((st = ensure(ctx, ctx->moe_h, n_pairs * d_ff * sizeof(float), s))) return st;
+        float *h = static_cast<float *>(ctx->moe_h.p), *u = nullptr;  // u (SwiGLU): the up products
+        if (w3) {
+            if ((st = ensure(ctx, ctx->moe_u, n_pairs * d_ff * sizeof(float), s))) return st;
+            u = static_cast<float *>(ctx->moe_u.p);
+        }
+        const size_t kmax = std::max(d_model, d_ff);
+        const size_t act_bytes = form == Q8_MFMA ? (size_t)max_tiles * gemv_q8_tile_bytes(kmax)
+                                                 : n_pairs * (kmax + kmax / 8 + kmax / 4);
+        if (mode == RCE_QMM_MODE_Q8 && (st = ensure(ctx, ctx->act_q, act_bytes, s))) return st;
+        if (mode == RCE_QMM_MODE_EXACT && (st = ensure(ctx, ctx->moe_x, n_pairs * d_model * sizeof(float), s))) return st;
+        HIP_TRY(launch_moe_group(ids_dev, n_pairs, (int)top_k, (int)n_expert, bm, offs, slot_of_pair, tok_of_slot, tiles,
+                                 n_tiles, status, ctx->moe_status, bases, nullptr, nullptr, 0, s));
+        HIP_TRY(hipEventRecord(ctx->moe_grouped, s));
+        const int act = w3 ? Q8SRC_SWIGLU : Q8SRC_SILU;
+        if (form == Q8_MFMA) {
+            void *q = ctx->act_q.p;
+            HIP_TRY(launch_quantize_tiles(Q8SRC_ROWS, x_dev, nullptr, d_model, 0, max_tiles, tiles, n_tiles, tok_of_slot, q, s));
+            HIP_TRY(launch_gemv_q8_grouped(a1, wtab1, h, w3 ? wtab3 : nullptr, u, q, max_tiles, tiles, n_tiles, s));
+            HIP_TRY(launch_quantize_tiles(act, h, u, d_ff, 0, max_tiles, tiles, n_tiles, nullptr, q, s));
+            HIP_TRY(launch_gemv_q8_grouped(a2, wtab2, y, nullptr, nullptr, q, max_tiles, tiles, n_tiles, s));
+        } else {
+            MoeGroup m;
+            m.wtab = wtab1;
+            m.wtab2 = w3 ? wtab3 : nullptr;
+            m.out2 = u;
+            m.tiles = tiles;
+            m.n_tiles = n_tiles;
+            m.max_tiles = max_tiles;
+            m.tb = bm;
+            m.n_slots_max = (int)n_pairs;
+            const bool q8 = mode == RCE_QMM_MODE_Q8;
+            void *q = q8 ? ctx->act_q.p : ctx->moe_x.p;
+            if (q8) HIP_TRY(launch_quantize_slots(Q8SRC_ROWS, x_dev, nullptr, d_model, (int)n_pairs, n_slots, tok_of_slot, q, s));
+            else HIP_TRY(launch_gather_rows(x_dev, tok_of_slot, n_slots, n_pairs, d_model, static_cast<float *>(q), s));
+            HIP_TRY(launch_gemv_grouped(a1, m, q, h, (int)mode, s));
+            if (q8) HIP_TRY(launch_quantize_slots(act, h, u, d_ff, (int)n_pairs, n_slots, nullptr, q, s));
+            else if (w3) HIP_TRY(launch_swiglu_slots(h, u, n_slots, n_pairs, d_ff, s));
+            else HIP_TRY(launch_silu_inplace(h, n_slots, n_pairs, d_ff, s));
+            m.wtab = wtab2;
+            m.wtab2 = nullptr;
+            m.out2 = nullptr;
+            HIP_TRY(launch_gemv_grouped(a2, m, q8 ? q : h, y, (int)mode, s));
+        }
+        HIP_TRY(launch_moe_combine(y, slot_of_pair, weights_dev, t_rows, (int)top_k, d_model, out_dev, s));
+        HIP_TRY(hipEventSynchronize(ctx->moe_grouped));
+        if (*static_cast<volatile int *>(ctx->moe_status)) return fail(RCE_QMM_BAD_SHAPE, "an expert id is out of range");
+        return RCE_QMM_OK;
     } else {
         if (mode != RCE_QMM_MODE_EXACT && mode != RCE_QMM_MODE_Q8) return fail(RCE_QMM_BAD_SHAPE, "unknown mode");
         HIP_TRY(launch_moe_group(ids_dev, n_pairs, (int)top_k, (int)n_expert, bm, offs, slot_of_pair, tok_of_slot,
-                                 tiles, n_tiles, status, nullptr, nullptr, 0, s));
+                                 tiles, n_tiles, status, nullptr, bases, nullptr, nullptr, 0, s));
         if ((st = ensure(ctx, ctx->moe_h, n_pairs * d_ff * sizeof(float), s))) return st;
         float *h = static_cast<float *>(ctx->moe_h.p);
         float *u = nullptr;  // SwiGLU: the up products

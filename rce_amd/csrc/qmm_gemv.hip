@@ -180,6 +180,41 @@ __global__ __launch_bounds__(64) void k_quantize_act(const float *__restrict__ A
     quant_task_finish<false>(q, k, total, task, L);
 }
 
+// The Q8 activations of a grouped call's slots, in the layout ActLds gives a
+// block of T tokens: of the slots' tokens' rows of A, or of silu(A) or
+// silu(A) * A2 of the slots themselves (the reference's form, as
+// k_swiglu_slots forms it).
+template <int SRC>
+__global__ __launch_bounds__(64) void k_quantize_slots(const float *__restrict__ A, const float *__restrict__ A2, size_t k,
+                                                       int T, const int *__restrict__ n_slots,
+                                                       const int *__restrict__ tok_of_slot, unsigned char *__restrict__ ws) {
+    const int slot = blockIdx.y, kq = (int)(k / 8);
+    if (slot >= n_slots[0]) return;
+    const int i = blockIdx.x * 64 + threadIdx.x;  // 8 values of the slot's row; past the row: its first ones, not stored
+    const int ii = i < kq ? i : 0;
+    const size_t row = SRC == Q8SRC_ROWS ? (size_t)tok_of_slot[slot] : (size_t)slot;
+    const float4 *p = reinterpret_cast<const float4 *>(A + row * k + 8 * (size_t)ii);
+    QuantTask q;
+    q.v0 = p[0];
+    q.v1 = p[1];
+    if constexpr (SRC != Q8SRC_ROWS) {
+        float4 u0 = make_float4(1.0f, 1.0f, 1.0f, 1.0f), u1 = u0;
+        if constexpr (SRC == Q8SRC_SWIGLU) {
+            const float4 *pu = reinterpret_cast<const float4 *>(A2 + row * k + 8 * (size_t)ii);
+            u0 = pu[0];
+            u1 = pu[1];
+        }
+        auto h = [](float g, float u) { return SRC == Q8SRC_SWIGLU ? silu_ref(g) * u : silu_ref(g); };
+        q.v0 = make_float4(h(q.v0.x, u0.x), h(q.v0.y, u0.y), h(q.v0.z, u0.z), h(q.v0.w, u0.w));
+        q.v1 = make_float4(h(q.v1.x, u1.x), h(q.v1.y, u1.y), h(q.v1.z, u1.z), h(q.v1.w, u1.w));
+    }
+    ActLds L(ws, k, T);
+    L.xq += (size_t)slot * k / 4;
+    L.dx += (size_t)slot * (k / 32);
+    L.s16 += (size_t)slot * (k / 16);
+    quant_task_finish<false>(q, k, kq, i, L);
+}
+
 }  // namespace
 
 // Column units per row must fit one block of up to 1024 threads.
@@ -742,6 +777,50 @@ hipError_t launch_gemv_q8_pre(const DevWeight &w, const float *a, size_t t_rows,
     case T_Q4_K: return launch_as_preq_tb<Q4_KQ8, 4>(w, g, a, t_rows, out, q, s);
     case T_Q5_K: return launch_as_preq_tb<Q5_KQ8, 4>(w, g, a, t_rows, out, q, s);
     case T_Q6_K: return launch_as_preq_tb<Q6_KQ8, 2>(w, g, a, t_rows, out, q, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_quantize_slots(int src, const float *a, const float *a2, size_t k, int n_slots_max, const int *n_slots,
+                                 const int *tok_of_slot, void *ws, hipStream_t s) {
+    const dim3 grid((unsigned)((k / 8 + 63) / 64), (unsigned)n_slots_max);
+    if (n_slots_max < 1 || n_slots_max > 65535) return hipErrorInvalidValue;
+    unsigned char *q = static_cast<unsigned char *>(ws);
+    if (src == Q8SRC_ROWS)
+        hipLaunchKernelGGL(k_quantize_slots<Q8SRC_ROWS>, grid, dim3(64), 0, s, a, a2, k, n_slots_max, n_slots, tok_of_slot, q);
+    else if (src == Q8SRC_SILU)
+        hipLaunchKernelGGL(k_quantize_slots<Q8SRC_SILU>, grid, dim3(64), 0, s, a, a2, k, n_slots_max, n_slots, tok_of_slot, q);
+    else
+        hipLaunchKernelGGL(k_quantize_slots<Q8SRC_SWIGLU>, grid, dim3(64), 0, s, a, a2, k, n_slots_max, n_slots, tok_of_slot, q);
+    return hipGetLastError();
+}
+
+// The formats on the activation-stationary kernel with a row in a block of
+// 512 threads (and Q6_K EXACT, its helper-wave kernel).
+bool gemv_grouped_supports(uint32_t dtype, size_t n_cols, int mode) {
+    if (!gpu_supports(dtype, n_cols, mode)) return false;
+    switch (dtype) {
+    case T_Q4_0: case T_Q8_0: case T_Q5_0: case T_Q4_1: case T_Q3_K: case T_Q4_K: case T_Q5_K: break;
+    case T_Q6_K:
+        if (mode == 0) return n_cols <= 16384;
+        break;
+    default: return false;
+    }
+    const int U = units_per_row(dtype, n_cols), nt = nt_for(U);
+    return nt <= 512 && gemv_lds_bytes(U, nt, 2, 2, false, n_cols) <= LDS_MAX;
+}
+
+hipError_t launch_gemv_grouped(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s) {
+    if (!gemv_grouped_supports(w.dtype, w.n_cols, mode) || m.max_tiles < 1 || m.max_tiles > 65535) return hipErrorInvalidValue;
+    switch (w.dtype) {
+    case T_Q4_0: return launch_gemv_grouped_q4_0(w, m, a, out, mode, s);
+    case T_Q8_0: return launch_gemv_grouped_q8_0(w, m, a, out, mode, s);
+    case T_Q4_K: return launch_gemv_grouped_q4_k(w, m, a, out, mode, s);
+    case T_Q5_K: return launch_gemv_grouped_q5_k(w, m, a, out, mode, s);
+    case T_Q6_K: return launch_gemv_grouped_q6_k(w, m, a, out, mode, s);
+    case T_Q5_0: return launch_gemv_grouped_q5_0(w, m, a, out, mode, s);
+    case T_Q4_1: return launch_gemv_grouped_q4_1(w, m, a, out, mode, s);
+    case T_Q3_K: return launch_gemv_grouped_q3_k(w, m, a, out, mode, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -1311,6 +1311,8 @@ __global__ __launch_bounds__(NT) void k_gemv_as(DevWeight w, const float *__rest
     constexpr int KIND = FX & 7;
     constexpr bool NORM = (FX & FX_NORM) != 0;
     constexpr bool PREQ = (FX & FX_PREQ) != 0;
+    constexpr bool GROUP = (FX & FX_GROUP) != 0;
+    static_assert(!GROUP || (KIND == 0 && !NORM && Q8 == PREQ), "grouped experts: plain launches, Q8 pre-quantized");
     static_assert(!PREQ || (Q8 && KIND == 0 && !NORM), "pre-quantized activations: plain Q8 launches");
     static_assert(!NORM || TB == 1, "the normalizing forms are single-token");
     extern __shared__ __align__(16) unsigned char lds[];
@@ -1335,8 +1337,15 @@ __global__ __launch_bounds__(NT) void k_gemv_as(DevWeight w, const float *__rest
     static_assert(KIND != FX_SWIGLU || RPL % 2 == 0, "swiglu pairs need an even row count per lane");
     const int RTO = KIND == FX_SWIGLU ? RT / 2 : RT;  // output rows of the block
     const size_t row0 = (size_t)bx * RTO;
-    const int t0 = blockIdx.y * TB;
-    const int tv = min(TB, t_rows - t0);
+    int t0 = blockIdx.y * TB, tv = min(TB, t_rows - t0);
+    if constexpr (GROUP) {
+        if ((int)blockIdx.y >= fx.n_tiles[0]) return;
+        const MoeTile tl = fx.tiles[blockIdx.y];
+        w = blockIdx.z ? fx.wtab2[tl.e] : fx.wtab[tl.e];
+        if (blockIdx.z) out = fx.out2;
+        t0 = tl.r0;
+        tv = tl.rows;
+    }
     const size_t k = w.n_cols;
 
     Unit unit;
@@ -1673,6 +1682,57 @@ hipError_t launch_as_preq_tb(const DevWeight &w, const GemvGeom &g, const float 
     default: return hipErrorInvalidValue;
     }
 #undef RCE_PQ
+}
+
+// Grouped experts (FX_GROUP): one or two slots per block; the most rows per
+// lane (8, 4, 2) whose addends fit the LDS and that leave two blocks per CU
+// when every tile is present.
+template <class Unit, int NT, int RPL, bool Q8>
+hipError_t launch_as_grouped(const DevWeight &w, int U, const MoeGroup &m, const void *a, float *out, hipStream_t s) {
+    constexpr int TB = Unit::NTOK;
+    const int P = NT / U, RT = P * RPL;
+    if (P < 1) return hipErrorInvalidConfiguration;
+    if (!wbuf_span_ok(w, RT)) return hipErrorInvalidValue;
+    const size_t lds = gemv_lds_bytes(U, NT, RPL, TB, false, w.n_cols);
+    if (lds > LDS_MAX) return hipErrorInvalidConfiguration;
+    GemvFx fx{};
+    fx.wtab = m.wtab;
+    fx.wtab2 = m.wtab2;
+    fx.out2 = m.out2;
+    fx.tiles = m.tiles;
+    fx.n_tiles = m.n_tiles;
+    fx.preq = Q8 ? static_cast<const unsigned char *>(a) : nullptr;
+    fx.preq_t = m.n_slots_max;
+    const dim3 grid((unsigned)((w.n_rows + RT - 1) / RT), (unsigned)m.max_tiles, m.wtab2 ? 2u : 1u);
+    constexpr int FX = FX_GROUP | (Q8 ? FX_PREQ : 0);
+    hipLaunchKernelGGL((k_gemv_as<Unit, NT, RPL, Q8, FX>), grid, dim3(NT), lds, s, w, static_cast<const float *>(a), out,
+                       m.n_slots_max, U, fx);
+    return hipGetLastError();
+}
+
+template <class Unit, bool Q8>
+hipError_t launch_as_grouped_nt(const DevWeight &w, const MoeGroup &m, const void *a, float *out, hipStream_t s) {
+    const int U = units_per_row(w.dtype, w.n_cols), nt = nt_for(U);
+    int rpl = 8;
+    auto blocks = [&](int r) { return (w.n_rows + (size_t)(nt / U) * r - 1) / ((size_t)(nt / U) * r) * (size_t)m.max_tiles; };
+    while (rpl > 2 && (gemv_lds_bytes(U, nt, rpl, Unit::NTOK, false, w.n_cols) > LDS_MAX || blocks(rpl) < 512)) rpl /= 2;
+#define RCE_GRP(NT)                                                              \
+    switch (rpl) {                                                               \
+    case 8: return launch_as_grouped<Unit, NT, 8, Q8>(w, U, m, a, out, s);       \
+    case 4: return launch_as_grouped<Unit, NT, 4, Q8>(w, U, m, a, out, s);       \
+    default: return launch_as_grouped<Unit, NT, 2, Q8>(w, U, m, a, out, s);      \
+    }
+    if (nt == 256) { RCE_GRP(256) }
+    if (nt == 512) { RCE_GRP(512) }
+    return hipErrorInvalidValue;
+#undef RCE_GRP
+}
+
+template <template <int> class Unit, bool Q8>
+hipError_t launch_as_grouped_tb(const DevWeight &w, const MoeGroup &m, const void *a, float *out, hipStream_t s) {
+    if (m.tb == 1) return launch_as_grouped_nt<Unit<1>, Q8>(w, m, a, out, s);
+    if (m.tb == 2) return launch_as_grouped_nt<Unit<2>, Q8>(w, m, a, out, s);
+    return hipErrorInvalidValue;
 }
 
 // MAXTB: the most tokens per thread the unit's registers allow.

@@ -197,7 +197,19 @@ enum : int { FX_SEG = 1, FX_RESIDUAL = 2, FX_SWIGLU = 3, FX_NORM = 8 };
 // GemvFx::preq (launch_gemv_q8_pre); blocks read their tokens' slices.
 constexpr int FX_PREQ = 16;
 
+// Grouped experts: blockIdx.y is a tile of tiles[0 .. n_tiles[0]), the slots
+// r0 .. r0 + rows - 1 of expert e, whose weight is wtab[e] (blockIdx.z = 1:
+// wtab2[e], output out2).
+constexpr int FX_GROUP = 32;
+
+struct MoeTile {
+    int e, r0, rows, pad;
+};
+
 struct GemvFx {
+    const struct DevWeight *wtab, *wtab2;  // FX_GROUP
+    const MoeTile *tiles;                  // FX_GROUP
+    const int *n_tiles;                    // FX_GROUP
     DevWeight w2, w3;      // FX_SEG: segments 1 and 2; FX_SWIGLU: w2 = up
     float *out2, *out3;    // FX_SEG: their outputs
     unsigned blk2, blk3;   // FX_SEG: first block of segments 1 and 2
@@ -385,10 +397,6 @@ hipError_t launch_f32_to_f16(const float *src, void *dst, size_t n, hipStream_t 
 
 // ---- grouped experts (moe.hip, gemm_f16.hip) ----
 // A row tile of the grouped GEMM: expert e, slots r0 .. r0 + rows - 1.
-struct MoeTile {
-    int e, r0, rows, pad;
-};
-
 // Which output tile (row tile mt, column tile nt) block blockIdx.x of a
 // prefill GEMM computes; false: none (the block returns before any barrier).
 // Blocks are dispatched round-robin over the 8 XCDs (block L to XCD L % 8),
@@ -423,15 +431,56 @@ __device__ __forceinline__ bool tile_of_block(size_t n_rows, int m_tiles, const 
     return true;
 }
 #endif
+// The decode kernels over a grouped call's tiles (at most `tb` slots each, 1
+// or 2): out[slot] = wtab[expert] . a[slot] (and out2 with wtab2, a second
+// matrix of the same shape).  mode 0: a is f32 rows by slot; mode 1: the
+// slots' Q8 activations as launch_quantize_slots writes them (n_slots_max
+// rows).
+struct MoeGroup {
+    const DevWeight *wtab = nullptr, *wtab2 = nullptr;
+    float *out2 = nullptr;
+    const MoeTile *tiles = nullptr;
+    const int *n_tiles = nullptr;
+    int max_tiles = 0, tb = 1, n_slots_max = 0;
+};
+bool gemv_grouped_supports(uint32_t dtype, size_t n_cols, int mode);
+hipError_t launch_gemv_grouped(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+// Q8 activations of the slots (act_lds_bytes(k, n_slots_max) bytes at ws):
+// of a's rows by src as launch_quantize_tiles.
+hipError_t launch_quantize_slots(int src, const float *a, const float *a2, size_t k, int n_slots_max, const int *n_slots,
+                                 const int *tok_of_slot, void *ws, hipStream_t s);
+// Per-format launchers (gemv_<format>.hip).
+hipError_t launch_gemv_grouped_q4_0(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q8_0(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q4_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q5_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q6_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q5_0(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q4_1(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+hipError_t launch_gemv_grouped_q3_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s);
+// The expert matrices' addresses by value, for a grouped call of at most
+// MOE_ARG_EXPERTS experts: the grouping kernel writes the device table
+// tab[m * n_expert + e] = proto[m] at base[m * n_expert + e] itself, so a call
+// whose experts differ from the last one's (every layer of a model) needs no
+// copy and no wait.
+constexpr int MOE_ARG_EXPERTS = 64;
+struct MoeBases {
+    DevWeight proto[3];
+    const uint8_t *base[3 * MOE_ARG_EXPERTS];
+    DevWeight *tab;  // nullptr: no table to write
+    int n_mat;
+};
 // Stable grouping of pairs p = token * top_k + j by expert ids[p]:
 // offs[n_expert + 1], slot_of_pair[n_pairs] (-1: id out of range),
 // tok_of_slot[n_pairs], tiles[n_pairs / bm + n_expert] (bm-row pieces of
-// each expert's slots), n_tiles[1], status[1] (1: an id was out of range).
+// each expert's slots), n_tiles[1], status[1] (1: an id was out of range),
+// also stored to host_status (mapped host memory) when given.
 // With x16 non-null the same launch also writes x16[i] = binary16(x[i]),
 // i < n_x.
 hipError_t launch_moe_group(const int32_t *ids, size_t n_pairs, int top_k, int n_expert, int bm, int *offs,
                             int *slot_of_pair, int *tok_of_slot, MoeTile *tiles, int *n_tiles, int *status,
-                            const float *x, void *x16, size_t n_x, hipStream_t s);
+                            int *host_status, const MoeBases &bases, const float *x, void *x16, size_t n_x,
+                            hipStream_t s);
 // xg[s, :] = x[tok_of_slot[s], :] for s < n_slots (device count)
 hipError_t launch_gather_rows(const float *x, const int *tok_of_slot, const int *n_slots_dev, size_t max_slots,
                               size_t d, float *xg, hipStream_t s);

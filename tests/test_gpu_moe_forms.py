@@ -1,0 +1,78 @@
+"""GPU parity of the grouped experts' EXACT and Q8 forms without a host
+round trip: tiles of one and two slots on the decode kernels, tiles of 16 on
+the int8 matrix cores, over every format, one and two slots per expert,
+experts without slots, and the most experts whose table travels in the kernel
+arguments (64) and one more.  Bit for bit with the oracle's device-order
+restatement."""
+import numpy as np
+import pytest
+
+import oracle as O
+import rce_amd
+from rand_blocks import rand_blocks
+from rce_amd import Mode
+from test_gpu_moe import bit_equal, run_moe
+
+pytestmark = pytest.mark.gpu
+
+
+def experts(rng, dt, count, n, k):
+    if dt in (O.Q4_1, O.Q5_0, O.Q3_K):
+        return [rand_blocks(rng, dt, n, k) for _ in range(count)]
+    return [O.quantize((rng.standard_normal((n, k)) * 0.02).astype(np.float32), dt) for _ in range(count)]
+
+
+def check(ctx, dt, E, dm, dff, t, k, mode):
+    print(f"moe forms dtype={dt} E={E} d={dm} ff={dff} t={t} k={k} mode={mode}", flush=True)
+    rng = np.random.default_rng(dt * 100 + E + t)
+    w1, w2 = experts(rng, dt, E, dff, dm), experts(rng, dt, E, dm, dff)
+    x = rng.standard_normal((t, dm)).astype(np.float32)
+    ids, gw = rce_amd.moe_router(rng.standard_normal((t, E)).astype(np.float32), k)
+    got = run_moe(ctx, w1, w2, dt, dm, dff, x, ids, gw, mode)
+    want = O.moe_ffn(x, w1, w2, dt, dff, ids, gw, q8=mode == Mode.Q8, silu_dev=True)
+    assert bit_equal(got, want)
+
+
+@pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
+@pytest.mark.parametrize("dt", [O.Q4_0, O.Q8_0, O.Q5_0, O.Q4_1, O.Q3_K, O.Q4_K, O.Q5_K, O.Q6_K])
+@pytest.mark.parametrize("E,t,k", [(4, 1, 1), (4, 5, 2), (2, 9, 2)])  # tiles of one, of two (ragged), several per expert
+def test_formats(ctx, dt, E, t, k, mode):
+    check(ctx, dt, E, 512, 768, t, k, mode)
+
+
+@pytest.mark.parametrize("dt", [O.Q4_0, O.Q4_K, O.Q6_K])
+def test_q8_on_the_matrix_cores(ctx, monkeypatch, dt):
+    monkeypatch.setenv("RCE_QMM_Q8_MFMA", "2")
+    check(ctx, dt, 3, 512, 768, 37, 2, Mode.Q8)  # about 25 slots per expert: a full tile and a ragged one
+
+
+@pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
+@pytest.mark.parametrize("E", [64, 65])
+def test_expert_table_limits(ctx, E, mode):
+    check(ctx, O.Q4_0, E, 256, 256, 40, 3, mode)
+
+
+@pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
+def test_experts_change_between_calls(ctx, mode):
+    """Two expert sets alternately on one context (a model's layers)."""
+    for seed in (1, 2, 1):
+        rng = np.random.default_rng(seed)
+        w1, w2 = experts(rng, O.Q4_K, 4, 512, 256), experts(rng, O.Q4_K, 4, 256, 512)
+        x = rng.standard_normal((3, 256)).astype(np.float32)
+        ids, gw = rce_amd.moe_router(rng.standard_normal((3, 4)).astype(np.float32), 2)
+        got = run_moe(ctx, w1, w2, O.Q4_K, 256, 512, x, ids, gw, mode)
+        assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q4_K, 512, ids, gw, q8=mode == Mode.Q8, silu_dev=True))
+
+
+@pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
+def test_bad_id_is_an_error_and_the_next_call_is_clean(ctx, mode):
+    rng = np.random.default_rng(3)
+    w1, w2 = experts(rng, O.Q4_0, 4, 512, 256), experts(rng, O.Q4_0, 4, 256, 512)
+    x = rng.standard_normal((4, 256)).astype(np.float32)
+    ids, gw = rce_amd.moe_router(rng.standard_normal((4, 4)).astype(np.float32), 2)
+    bad = ids.copy()
+    bad[2, 1] = -1
+    with pytest.raises(rce_amd.QmmError, match="out of range"):
+        run_moe(ctx, w1, w2, O.Q4_0, 256, 512, x, bad, gw, mode)
+    got = run_moe(ctx, w1, w2, O.Q4_0, 256, 512, x, ids, gw, mode)
+    assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q4_0, 512, ids, gw, q8=mode == Mode.Q8, silu_dev=True))
