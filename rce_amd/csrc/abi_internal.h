@@ -30,6 +30,9 @@ inline rce_qmm_status hip_fail(hipError_t e, const char *what) {
         if (e_ != hipSuccess) return hip_fail(e_, #expr);   \
     } while (0)
 
+// Bytes of each of a context's two pinned staging buffers.
+constexpr size_t HOST_STAGE = 256 * 1024;
+
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // A device allocation shared by a weight and its views.
@@ -71,6 +74,10 @@ struct rce_qmm_context {
     // EXACT / Q8 grouped calls: the grouping kernel's status word in mapped
     // host memory, and the event after that kernel
     int *moe_status = nullptr;
+    // pinned staging of the host-pointer entry points (HOST_STAGE bytes each)
+    unsigned char *host_in = nullptr, *host_out = nullptr;
+    // mapped host word the last kernel of such a call sets to its number
+    uint32_t *host_done = nullptr, host_calls = 0;
     hipEvent_t moe_grouped = nullptr;
 };
 

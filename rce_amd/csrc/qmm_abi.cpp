@@ -9,6 +9,7 @@
 #include "lds_limit.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -196,6 +197,35 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
 
 namespace {
 
+// The context's pinned staging buffers, made at the first call that uses
+// them; false where they cannot be allocated.
+bool host_staging(rce_qmm_context *ctx) {
+    auto make = [](void **p, size_t bytes) {
+        if (*p) return true;
+        if (hipHostMalloc(p, bytes, hipHostMallocDefault) == hipSuccess) return true;
+        *p = nullptr;
+        (void)hipGetLastError();
+        return false;
+    };
+    if (!make(reinterpret_cast<void **>(&ctx->host_in), HOST_STAGE) || !make(reinterpret_cast<void **>(&ctx->host_out), HOST_STAGE))
+        return false;
+    if (!ctx->host_done) {
+        if (!make(reinterpret_cast<void **>(&ctx->host_done), 64)) return false;
+        *ctx->host_done = ctx->host_calls;
+    }
+    return true;
+}
+
+// Whether *flag became v within 200 us.
+bool poll_flag(const uint32_t *flag, uint32_t v) {
+    const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    do {
+        for (int i = 0; i < 64; i++)
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == v) return true;
+    } while (std::chrono::steady_clock::now() < end);
+    return false;
+}
+
 rce_qmm_status host_batched(rce_qmm_context *ctx, const float *a, size_t t_rows, const rce_qmm_weight *w,
                             float *out) {
     rce_qmm_status st = check_weight_ctx(ctx, w);
@@ -209,6 +239,25 @@ rce_qmm_status host_batched(rce_qmm_context *ctx, const float *a, size_t t_rows,
     if (t_rows == 0 || dw.n_rows == 0) return RCE_QMM_OK;
     const size_t abytes = t_rows * dw.n_cols * sizeof(float), obytes = t_rows * dw.n_rows * sizeof(float);
     if ((st = ensure(ctx, ctx->a_in, abytes, nullptr))) return st;
+    // Small calls through the context's pinned staging: a kernel fetches the
+    // activations over the bus, the product writes its rows straight into
+    // host memory and a last kernel sets a flag there, which the host polls
+    // (for a while: a long or failed call is left to the stream's own wait,
+    // which also reports errors).  Copies from and to the caller's pageable
+    // memory and the stream's wait take about 8 us each whatever the size.
+    // Larger calls keep the copies.
+    if (align_up(abytes, 16) <= HOST_STAGE && obytes <= HOST_STAGE && host_staging(ctx)) {
+        std::memcpy(ctx->host_in, a, abytes);
+        HIP_TRY(launch_copy16(ctx->host_in, ctx->a_in.p, (abytes + 15) / 16, ctx->stream));
+        if ((st = run_batched(ctx, ctx->a_in.p, T_F32, t_rows, w, reinterpret_cast<float *>(ctx->host_out),
+                              RCE_QMM_MODE_EXACT, ctx->stream, nullptr, 0)))
+            return st;
+        const uint32_t call = ++ctx->host_calls;
+        HIP_TRY(launch_host_flag(ctx->host_done, call, ctx->stream));
+        if (!poll_flag(ctx->host_done, call)) HIP_TRY(hipStreamSynchronize(ctx->stream));
+        std::memcpy(out, ctx->host_out, obytes);
+        return RCE_QMM_OK;
+    }
     if ((st = ensure(ctx, ctx->out, obytes, nullptr))) return st;
     HIP_TRY(hipMemcpyAsync(ctx->a_in.p, a, abytes, hipMemcpyHostToDevice, ctx->stream));
     if ((st = run_batched(ctx, ctx->a_in.p, T_F32, t_rows, w, static_cast<float *>(ctx->out.p), RCE_QMM_MODE_EXACT,
@@ -286,7 +335,8 @@ void rce_qmm_abi::context_release(rce_qmm_context *ctx) {
                        &ctx->moe_h, &ctx->moe_h16, &ctx->moe_y, &ctx->moe_u})
         if (s->p) (void)hipFree(s->p);
     if (ctx->moe_grouped) (void)hipEventDestroy(ctx->moe_grouped);
-    if (ctx->moe_status) (void)hipHostFree(ctx->moe_status);
+    for (void *p : {(void *)ctx->moe_status, (void *)ctx->host_in, (void *)ctx->host_out, (void *)ctx->host_done})
+        if (p) (void)hipHostFree(p);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

@@ -180,6 +180,15 @@ __global__ __launch_bounds__(64) void k_quantize_act(const float *__restrict__ A
     quant_task_finish<false>(q, k, total, task, L);
 }
 
+__global__ __launch_bounds__(256) void k_copy16(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n16) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n16) dst[i] = src[i];
+}
+
+__global__ void k_host_flag(uint32_t *flag, uint32_t v) {
+    __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The Q8 activations of a grouped call's slots, in the layout ActLds gives a
 // block of T tokens: of the slots' tokens' rows of A, or of silu(A) or
 // silu(A) * A2 of the slots themselves (the reference's form, as
@@ -779,6 +788,18 @@ hipError_t launch_gemv_q8_pre(const DevWeight &w, const float *a, size_t t_rows,
     case T_Q6_K: return launch_as_preq_tb<Q6_KQ8, 2>(w, g, a, t_rows, out, q, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_copy16(const void *src, void *dst, size_t n16, hipStream_t s) {
+    if (n16 == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_copy16, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, s, static_cast<const uint4 *>(src),
+                       static_cast<uint4 *>(dst), n16);
+    return hipGetLastError();
+}
+
+hipError_t launch_host_flag(uint32_t *flag, uint32_t v, hipStream_t s) {
+    hipLaunchKernelGGL(k_host_flag, dim3(1), dim3(1), 0, s, flag, v);
+    return hipGetLastError();
 }
 
 hipError_t launch_quantize_slots(int src, const float *a, const float *a2, size_t k, int n_slots_max, const int *n_slots,

@@ -310,6 +310,11 @@ size_t layout_pad_bytes(const DevWeight &dw);
 void relayout_host(const uint8_t *src, const DevWeight &dw, uint8_t *dst);
 
 hipError_t launch_f16_to_f32(const uint16_t *src, float *dst, size_t n, hipStream_t s);
+// dst[i] = src[i], i < n16 16-byte words (src in mapped host memory).
+hipError_t launch_copy16(const void *src, void *dst, size_t n16, hipStream_t s);
+// *flag (mapped host memory) = v, after everything before it on the stream is
+// visible to the host.
+hipError_t launch_host_flag(uint32_t *flag, uint32_t v, hipStream_t s);
 // mode 0: the reference's f32 order; mode 1: Q8 activations.  `geom`
 // overrides the shape the library picks (tuning only; nullptr = pick).
 hipError_t launch_gemv(const DevWeight &w, const float *a, size_t t_rows, float *out, int mode,
