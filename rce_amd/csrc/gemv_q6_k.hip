@@ -202,6 +202,286 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q6k_split(DevWeight w, const
     }
 }
 
+// ---------------------------------------------------------------------------
+// Q6_K Q8: a block owns R rows (R consecutive lanes of a 64-row group) and TB
+// tokens; thread (r = tid % R, sb = tid / R) forms the sum of super-block sb,
+// then sb + 256 / R, ... of row r, and the row's sums are folded in
+// super-block order (rce-op-qmm/src/lib.rs L1667-1705's order).  A load
+// instruction's R lanes read R * 16 contiguous bytes of one chunk plane, whole
+// lines, where the activation-stationary form (a lane per super-block of a
+// row, consecutive lanes a super-block apart) touched a line per lane for 16
+// bytes of it; and the activations stay in LDS (a super-block's 256 values
+// are one address for its R lanes) instead of 64 registers per token, so a
+// SIMD holds five or six waves instead of two.  Bound by the weight's bytes
+// at 32000x2048, by latency (quantize, barrier, 13 chunks, fold) below.
+// Measured (us, that form / this one): 2048x5632 at 1 / 2 / 4 / 8 tokens
+// 12.6 / 14.2 / 18.6 / 34.4 against 6.2 / 9.1 / 9.0 / 11.5; 32000x2048 at 1 / 2 /
+// 4 / 8 11.8 / 26 / 50 / 95 against 9.1 (5.9 TB/s, cache included) / 10.4 / 16.8 /
+// 28.8; 4096x14336 at 1 / 8 39 / 156 against 14.3 / 32.8.
+// FX: the decode step's fused forms and grouped experts, as in k_gemv_as
+// (FX_SWIGLU: lanes r < R / 2 gate rows, the others the same up rows).
+// ---------------------------------------------------------------------------
+template <int TB, int R, int FX>
+__global__ __launch_bounds__(256) void k_gemv_q8_q6k(DevWeight w, const float *__restrict__ A, float *__restrict__ out,
+                                                     int t_rows, GemvFx fx) {
+    constexpr int NT = 256, NS = NT / R, KIND = FX & 7;
+    constexpr bool NORM = (FX & FX_NORM) != 0, GROUP = (FX & FX_GROUP) != 0;
+    static_assert(64 % R == 0 && (!GROUP || FX == FX_GROUP) && (!NORM || TB == 1), "forms");
+    constexpr int RO = KIND == FX_SWIGLU ? R / 2 : R;  // output rows of the block
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x, r = tid % R, sb0 = tid / R;
+    unsigned bx = blockIdx.x;
+    if constexpr (KIND == FX_SEG) {  // block-uniform choice of the segment
+        if (fx.pos && bx == 0 && tid == 0 && fx.status[2] == 0) {  // the step's last kernel: advance the position
+            const int p = fx.pos[0];
+            if (p >= fx.ctx_len && fx.status[0] == 0) fx.status[0] = 2;
+            fx.pos[0] = p + 1;
+        }
+        if (bx >= fx.blk3) { w = fx.w3; out = fx.out3; bx -= fx.blk3; }
+        else if (bx >= fx.blk2) { w = fx.w2; out = fx.out2; bx -= fx.blk2; }
+    }
+    int t0 = blockIdx.y * TB, tv = min(TB, t_rows - t0);
+    if constexpr (GROUP) {
+        if ((int)blockIdx.y >= fx.n_tiles[0]) return;
+        const MoeTile tl = fx.tiles[blockIdx.y];
+        w = blockIdx.z ? fx.wtab2[tl.e] : fx.wtab[tl.e];
+        if (blockIdx.z) out = fx.out2;
+        t0 = tl.r0;
+        tv = tl.rows;
+    }
+    const size_t row0 = (size_t)bx * RO, k = w.n_cols;
+    const int nsb = (int)(k / 256);
+    // RO divides 64, so the block's rows lie in one 64-row group, which the
+    // layout holds whole: rows past n_rows are its padding.  Super-blocks
+    // past the row repeat its last; neither is folded.
+    const uint8_t *base = w.base;
+    if constexpr (KIND == FX_SWIGLU) base = r >= RO ? fx.w2.base : base;
+    base += (row0 / 64) * w.group_stride;
+    const size_t ln = (row0 & 63) + r % RO;
+    v4u32 c[13];
+    uint32_t dr;
+    auto load = [&](int sb) {
+        const uint8_t *sp = base + (size_t)min(sb, nsb - 1) * IL64_Q6K_SB;
+#pragma unroll
+        for (int j = 0; j < 13; j++)
+            c[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u32 *>(sp + ((size_t)j * 64 + ln) * 16));
+        dr = ldw2(sp + IL64_Q6K_D + ln * 2);
+    };
+    // the activations' loads go out first (they are waited for first)
+    const int kq = (int)(k / 8), total = GROUP ? 0 : tv * kq;
+    QuantTask q0, q1;
+    if constexpr (!GROUP) {
+        quant_task_load(A, kq, t0, total, tid, q0);
+        quant_task_load(A, kq, t0, total, tid + NT, q1);
+        if constexpr (NORM) {
+            quant_task_load_g(fx.norm_w, kq, total, tid, q0);
+            quant_task_load_g(fx.norm_w, kq, total, tid + NT, q1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    load(sb0);
+    __builtin_amdgcn_sched_barrier(0);
+    ActLds L(lds, k, TB);
+    if constexpr (GROUP) {
+        const ActLds G(const_cast<unsigned char *>(fx.preq), k, fx.preq_t);
+        for (int t = 0; t < tv; t++) {
+            const int4 *gx = reinterpret_cast<const int4 *>(G.xq + (size_t)(t0 + t) * (k / 4));
+            const int4 *gd = reinterpret_cast<const int4 *>(G.dx + (size_t)(t0 + t) * (k / 32));
+            const int4 *gs = reinterpret_cast<const int4 *>(G.s16 + (size_t)(t0 + t) * (k / 16));
+            int4 *lx = reinterpret_cast<int4 *>(L.xq + t * (k / 4)), *ld = reinterpret_cast<int4 *>(L.dx + t * (k / 32));
+            int4 *ls = reinterpret_cast<int4 *>(L.s16 + t * (k / 16));
+            for (int i = tid; i < (int)(k / 16); i += NT) lx[i] = gx[i];
+            for (int i = tid; i < (int)(k / 128); i += NT) ld[i] = gd[i];
+            for (int i = tid; i < (int)(k / 64); i += NT) ls[i] = gs[i];
+        }
+    } else {
+        float inv = 0.0f;
+        if constexpr (NORM) {  // rms_norm's scale from the whole row (kq <= 2 NT), as k_gemv_as
+            __shared__ float red[NT / 64];
+            float ss = quant_task_ssq(q0, tid < total);
+            ss = ss + quant_task_ssq(q1, tid + NT < total);
+            ss = wave_sum(ss);
+            if ((tid & 63) == 0) red[tid >> 6] = ss;
+            __syncthreads();
+            float tot = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NT / 64; i++) tot = tot + red[i];
+            const float mean_sq = tot / (float)k;
+            inv = 1.0f / sqrtf(mean_sq + fx.eps);
+        }
+        quant_task_finish<NORM>(q0, k, total, tid, L, inv);
+        quant_task_finish<NORM>(q1, k, total, tid + NT, L, inv);
+        for (int i = 2 * NT; i < total; i += NT) {
+            QuantTask q;
+            quant_task_load(A, kq, t0, total, i + tid, q);
+            quant_task_finish(q, k, total, i + tid, L);
+        }
+    }
+    __syncthreads();
+    // [super-block, padded to whole passes][token][row]: every lane stores, so
+    // no arithmetic is sunk into a branch
+    float *part = reinterpret_cast<float *>(lds + act_lds_bytes(k, TB));
+    for (int s0 = 0; s0 < nsb; s0 += NS) {
+        const int sb = min(s0 + sb0, nsb - 1);
+        RawQ6_K raw;
+        // the chunks enter the body as whole register quadruples: passed in
+        // word by word, the compiler reused their registers before the reads
+#pragma unroll
+        for (int j = 0; j < 13; j++) {
+            asm volatile("" : "+v"(c[j]));
+            raw.c[j] = make_uint4(c[j].x, c[j].y, c[j].z, c[j].w);
+        }
+        const float d = h2f(dr);
+        float ssb[TB];
+#pragma unroll
+        for (int t = 0; t < TB; t++) ssb[t] = 0.0f;
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            int acc[TB][8];  // sub-block 8 o + 2 m + h -> index 2 m + h
+#pragma unroll
+            for (int h = 0; h < 2; h++) {  // words 4 h .. 4 h + 3 of the half's quarters
+                asm volatile("" ::: "memory");  // only their activations in registers at a time
+                uint32_t u[4][4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) q6_words(raw, o, 4 * h + j, u[0][j], u[1][j], u[2][j], u[3][j]);
+#pragma unroll
+                for (int m = 0; m < 4; m++)
+#pragma unroll
+                    for (int t = 0; t < TB; t++) {
+                        const int4 x = *reinterpret_cast<const int4 *>(L.xq + t * (k / 4) + 64 * (size_t)sb + 32 * o +
+                                                                       8 * m + 4 * h);
+                        int a = __builtin_amdgcn_sdot4((int)u[m][0], x.x, 0, false);
+                        a = __builtin_amdgcn_sdot4((int)u[m][1], x.y, a, false);
+                        a = __builtin_amdgcn_sdot4((int)u[m][2], x.z, a, false);
+                        acc[t][2 * m + h] = __builtin_amdgcn_sdot4((int)u[m][3], x.w, a, false);
+                    }
+            }
+#pragma unroll
+            for (int bb = 0; bb < 8; bb++) {  // sub-blocks in order: s += (d sc) (dx (dot - 32 sum))
+                const int sbk = 8 * o + bb;
+                const float ds = d * (float)q6_sc(raw.c[12], sbk);
+#pragma unroll
+                for (int t = 0; t < TB; t++) {
+                    const int isum = acc[t][bb] - 32 * L.s16[t * (k / 16) + 16 * (size_t)sb + sbk];
+                    const float ab = L.dx[t * (k / 32) + 8 * (size_t)sb + (sbk >> 1)] * (float)isum;
+                    ssb[t] = ssb[t] + ds * ab;
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TB; t++) part[((s0 + sb0) * TB + t) * R + r] = ssb[t];
+        asm volatile("" ::: "memory");  // the next loads go into the registers just used
+        if (s0 + NS < nsb) load(s0 + NS + sb0);
+    }
+    __syncthreads();
+    auto fold = [&](int t, int rr) {
+        float s = 0.0f;
+#pragma unroll 8
+        for (int sb = 0; sb < nsb; sb++) s = s + part[(sb * TB + t) * R + rr];
+        return s;
+    };
+    for (int j = tid; j < tv * RO; j += NT) {
+        const int t = j / RO, rr = j % RO;
+        if (row0 + rr < w.n_rows) {
+            const size_t o = ((size_t)t0 + t) * w.n_rows + row0 + rr;
+            if constexpr (KIND == FX_SWIGLU) {
+                const float g = fold(t, rr), u = fold(t, RO + rr);
+                out[o] = silu_ref(g) * u;  // rce-tinyllama L320: h = silu(g) * u
+            } else if constexpr (KIND == FX_RESIDUAL) {
+                out[o] = fx.res[o] + fold(t, rr);  // rce-tinyllama L318, L323: x += ...
+            } else {
+                out[o] = fold(t, rr);
+            }
+        }
+    }
+}
+
+size_t q6_q8_lds(size_t k, int tb, int r) {
+    const size_t ns = 256 / (size_t)r;
+    return act_lds_bytes(k, tb) + (k / 256 + ns - 1) / ns * ns * tb * r * sizeof(float);
+}
+
+// Rows per block: 16 spreads a row's super-blocks over 16 threads, 32 halves
+// the blocks' repeated quantization and activation staging, so 32 where it
+// still leaves two blocks per CU.  `units` is tokens / TB (times matrices).
+// Measured, 16 / 32 rows (us, a separate quantization launch of about 3
+// included): 512 blocks of 32 rows: 4096x4096 at 8 tokens 14.6 / 13.0, 4096x14336
+// at 8 46 / 37; 256 blocks: 4096x4096 at 4 10.4 / 11.0, 4096x14336 at 4 28 / 28.
+bool q6_rows32(size_t n_rows, size_t k, int tb, size_t units) {
+    return (n_rows + 31) / 32 * units >= 512 && q6_q8_lds(k, tb, 32) <= LDS_MAX;
+}
+
+template <int TB, int R, int FX>
+hipError_t launch_q6_q8(const DevWeight &w, const float *a, size_t t_rows, float *out, const GemvFx &fx, dim3 grid,
+                        hipStream_t s) {
+    const size_t lds = q6_q8_lds(w.n_cols, TB, R);  // 16 rows, two tokens, the longest row (act_lds_bytes(k, 1) = LDS_MAX): 151 KB
+    if (lds > LDS_MAX) {
+        const hipError_t e = ensure_lds_limit((const void *)k_gemv_q8_q6k<TB, R, FX>, 160 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_gemv_q8_q6k<TB, R, FX>), grid, dim3(256), lds, s, w, a, out, (int)t_rows, fx);
+    return hipGetLastError();
+}
+
+template <int TB>
+hipError_t launch_q6_q8_plain(const DevWeight &w, const float *a, size_t t_rows, float *out, hipStream_t s) {
+    const size_t tg = (t_rows + TB - 1) / TB;
+    if (q6_rows32(w.n_rows, w.n_cols, TB, tg))
+        return launch_q6_q8<TB, 32, 0>(w, a, t_rows, out, GemvFx{}, dim3((unsigned)((w.n_rows + 31) / 32), (unsigned)tg), s);
+    return launch_q6_q8<TB, 16, 0>(w, a, t_rows, out, GemvFx{}, dim3((unsigned)((w.n_rows + 15) / 16), (unsigned)tg), s);
+}
+
+template <int TB>
+hipError_t launch_q6_q8_grouped(const DevWeight &w, const MoeGroup &m, const void *a, float *out, hipStream_t s) {
+    GemvFx fx{};
+    fx.wtab = m.wtab;
+    fx.wtab2 = m.wtab2;
+    fx.out2 = m.out2;
+    fx.tiles = m.tiles;
+    fx.n_tiles = m.n_tiles;
+    fx.preq = static_cast<const unsigned char *>(a);
+    fx.preq_t = m.n_slots_max;
+    const unsigned y = (unsigned)m.max_tiles, z = m.wtab2 ? 2u : 1u;
+    if (q6_rows32(w.n_rows, w.n_cols, TB, (size_t)y * z))
+        return launch_q6_q8<TB, 32, FX_GROUP>(w, nullptr, 0, out, fx, dim3((unsigned)((w.n_rows + 31) / 32), y, z), s);
+    return launch_q6_q8<TB, 16, FX_GROUP>(w, nullptr, 0, out, fx, dim3((unsigned)((w.n_rows + 15) / 16), y, z), s);
+}
+
+// The decode step's fused forms (launch_gemv_fx has checked dtypes, columns
+// and the normalizing forms' row length).
+template <int FX>
+hipError_t launch_q6_q8_fx(const FxLaunch &f, const float *a, hipStream_t s) {
+    GemvFx fx{};
+    fx.norm_w = f.norm_w;
+    fx.eps = f.eps;
+    fx.pos = f.pos;
+    fx.status = f.status;
+    fx.ctx_len = f.ctx_len;
+    fx.res = f.res;
+    constexpr bool SEG = (FX & 7) == FX_SEG, PAIR = (FX & 7) == FX_SWIGLU;
+    if (f.pos && (!SEG || !f.status)) return hipErrorInvalidValue;
+    if ((FX & FX_NORM) && !f.norm_w) return hipErrorInvalidValue;
+    size_t rows = f.w[0].n_rows;
+    if (SEG)
+        for (int i = 1; i < f.nw; i++) rows += f.w[i].n_rows;
+    const bool r32 = q6_rows32(PAIR ? 2 * rows : rows, f.w[0].n_cols, 1, 1);
+    const size_t ro = (r32 ? 32 : 16) / (PAIR ? 2 : 1);
+    auto nblk = [&](const DevWeight &w) { return (unsigned)((w.n_rows + ro - 1) / ro); };
+    unsigned blocks = nblk(f.w[0]);
+    fx.blk2 = fx.blk3 = ~0u;
+    if (SEG) {
+        if (f.nw < 1 || f.nw > 3) return hipErrorInvalidValue;
+        if (f.nw >= 2) { fx.w2 = f.w[1]; fx.out2 = f.out[1]; fx.blk2 = blocks; blocks += nblk(f.w[1]); }
+        if (f.nw >= 3) { fx.w3 = f.w[2]; fx.out3 = f.out[2]; fx.blk3 = blocks; blocks += nblk(f.w[2]); }
+    }
+    if (PAIR) {
+        if (f.nw != 2 || f.w[1].n_rows != f.w[0].n_rows) return hipErrorInvalidValue;
+        fx.w2 = f.w[1];
+    }
+    return r32 ? launch_q6_q8<1, 32, FX>(f.w[0], a, 1, f.out[0], fx, dim3(blocks), s)
+               : launch_q6_q8<1, 16, FX>(f.w[0], a, 1, f.out[0], fx, dim3(blocks), s);
+}
+
 size_t q6_split_lds(size_t k) { return (k + 4) * sizeof(float) + 2 * 96 * 64 * sizeof(float); }
 
 hipError_t launch_q6_split(const DevWeight &w, const float *a, size_t t_rows, float *out, hipStream_t s) {
@@ -224,7 +504,10 @@ hipError_t q6_prepare_lds() {
 }
 
 hipError_t launch_gemv_grouped_q6_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s) {
-    if (mode != 0) return launch_as_grouped_tb<Q6_KQ8, true>(w, m, a, out, s);
+    if (mode != 0) {
+        if (m.tb == 1) return launch_q6_q8_grouped<1>(w, m, a, out, s);
+        return m.tb == 2 ? launch_q6_q8_grouped<2>(w, m, a, out, s) : hipErrorInvalidValue;
+    }
     if (w.n_cols > Q6_EXACT_LDS_K) return hipErrorInvalidValue;
     const size_t lds = q6_split_lds(w.n_cols);
     if (lds > 64 * 1024) {
@@ -241,7 +524,7 @@ hipError_t launch_gemv_grouped_q6_k(const DevWeight &w, const MoeGroup &m, const
     return hipSuccess;
 }
 
-hipError_t launch_gemv_q6_k(const DevWeight &w, const GemvGeom &g, const float *a, size_t t_rows, float *out, int mode,
+hipError_t launch_gemv_q6_k(const DevWeight &w, const float *a, size_t t_rows, float *out, int mode,
                             hipStream_t s) {
     if (mode == 0) {
         if (w.n_cols <= Q6_EXACT_LDS_K) return launch_q6_split(w, a, t_rows, out, s);
@@ -249,10 +532,21 @@ hipError_t launch_gemv_q6_k(const DevWeight &w, const GemvGeom &g, const float *
         hipLaunchKernelGGL(k_gemv_exact_q6k, grid, dim3(256), 0, s, w, a, out);
         return hipGetLastError();
     }
-    return launch_as_tb<Q6_KQ8, true, 2>(w, g, a, t_rows, out, s);
+    // one token or two per block: four hold the block's LDS and registers for
+    // the gain of a weight read from the Infinity Cache (us, two / four per
+    // block at 4 tokens: 4096x4096 10.4 / 11.1, 2048x5632 11.9 / 15.8,
+    // 32000x2048 20.5 / 18.9)
+    return t_rows == 1 ? launch_q6_q8_plain<1>(w, a, t_rows, out, s) : launch_q6_q8_plain<2>(w, a, t_rows, out, s);
 }
-hipError_t launch_gemv_fx_q6_k(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s) {
+hipError_t launch_gemv_fx_q6_k(const FxLaunch &f, const float *a, int mode, hipStream_t s) {
     if (mode == 0) return hipErrorInvalidValue;  // EXACT Q6_K is one lane per row
-    return launch_as_fx_nt<Q6_KQ8<1>, true>(f, g, a, s);
+    switch (f.kind) {
+    case FX_SEG: return launch_q6_q8_fx<FX_SEG>(f, a, s);
+    case FX_SEG | FX_NORM: return launch_q6_q8_fx<FX_SEG | FX_NORM>(f, a, s);
+    case FX_RESIDUAL: return launch_q6_q8_fx<FX_RESIDUAL>(f, a, s);
+    case FX_SWIGLU: return launch_q6_q8_fx<FX_SWIGLU>(f, a, s);
+    case FX_SWIGLU | FX_NORM: return launch_q6_q8_fx<FX_SWIGLU | FX_NORM>(f, a, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 }  // namespace rce_qmm

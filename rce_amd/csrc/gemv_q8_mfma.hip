@@ -4,7 +4,7 @@
 // integers with a token's Q8 integers is one lane's element of a
 // v_mfma_i32_16x16x32_i8 (16 weight rows x 16 tokens, K = one block), and
 // the rest is the decode kernels' f32 arithmetic in their order
-// (qmm_gemv_kernels.h: Q32Q8, Q4_KQ8, Q5_KQ8, Q6_KQ8), the row sum folded
+// (qmm_gemv_kernels.h: Q32Q8, Q4_KQ8, Q5_KQ8; gemv_q6_k.hip), the row sum folded
 // over units in order from +0.0 in registers.  So the result is bit-identical
 // to the decode kernels' Q8 mode and to the oracle's orc_mm_batched_q8.
 //
@@ -562,18 +562,19 @@ bool gemv_q8_mfma_supports(uint32_t dtype, size_t n_cols, size_t t_rows) {
 // Where this form is the faster one, by estimates fitted to both forms'
 // times (us, quantization included) at 2-64 tokens, N 1024-14336, K
 // 2048-8192.  With M = N K / 10^6 and tiles of 16 tokens:
-//   decode kernels: 7.3 + 0.021 M per token; Q6_K 8 + 0.16 M (two tokens per
+//   decode kernels: 7.3 + 0.021 M per token; Q6_K 5 + 0.05 M (two tokens per
 //     block, and its super-block's scales per token); a row of more than 256
 //     units (blocks of 32: K > 8192, 64-groups: K > 16384) 4 + 0.2 M from 4
 //     tokens on (no pre-quantized form there);
 //   this form: the larger of its chain over K, 5 + 1.2 (K-quants), 1.6
 //     (blocks of 32), 2.7 (Q6_K) per 1024 of K, and its arithmetic, 5 + 0.18 M
-//     (Q6_K 0.41) per tile.
+//     (Q6_K 0.43) per tile.
 // Measured there, decode kernels / this form: Q4_K 14336x4096 at 8 / 16 / 32 /
 // 64 tokens 19.2 / 28.2 / 47.4 / 87.9 against 17.9 / 18.3 / 25.9 / 44.2; Q4_0
 // 11008x4096 at 8 / 16 / 32 14.0 / 20.7 / 33.4 against 15.6 / 15.8 / 24.2; Q4_0
 // 4096x14336 at 4 / 16 / 64 50 / 183 / 739 against 28 / 28 / 48; Q6_K 2048x5632
-// at 4 / 8 / 32 18.6 / 34.5 / 95 against 20 / 20 / 21; Q8_0 512x8192 at 32
+// at 8 / 24 / 32 11.5 / 18.5 / 22.0 against 20.2 / 20.6 / 20.6, 11008x4096 at 8 /
+// 12 / 32 24.6 / 33.0 / 76 against 25.2 / 25.4 / 41; Q8_0 512x8192 at 32
 // 10.3 against 17.7.
 // RCE_QMM_Q8_MFMA: 0 = never this form, 2 = always where it applies (tests of
 // both forms on the same shapes).  Read at every call, so a test can switch it.
@@ -583,10 +584,10 @@ bool gemv_q8_mfma_preferred(const DevWeight &w, size_t t_rows) {
     if (mode != 1) return mode == 2;
     const double m = (double)w.n_rows * (double)w.n_cols * 1e-6, t = (double)t_rows, k = (double)w.n_cols / 1024.0;
     const bool q6 = w.dtype == T_Q6_K, kq = w.dtype == T_Q4_K || w.dtype == T_Q5_K;
-    const double decode = q6 ? 8.0 + 0.16 * m * t
+    const double decode = q6 ? 5.0 + 0.05 * m * t
                              : nt_for(units_per_row(w.dtype, w.n_cols)) != 256 && t_rows >= 4 ? 4.0 + 0.2 * m * t
                                                                                             : 7.3 + 0.021 * m * t;
-    const double chain = (q6 ? 2.7 : kq ? 1.2 : 1.6) * k, work = (q6 ? 0.41 : 0.18) * m * (double)((t_rows + 15) / 16);
+    const double chain = (q6 ? 2.7 : kq ? 1.2 : 1.6) * k, work = (q6 ? 0.43 : 0.18) * m * (double)((t_rows + 15) / 16);
     return 5.0 + (chain > work ? chain : work) < decode;
 }
 

@@ -544,14 +544,15 @@ namespace {
 
 // Q8 grouped experts: the int8 matrix cores (tiles of 16 slots, whatever they
 // hold) against the decode kernels over tiles of two slots.  Measured (us,
-// decode / matrix cores, 8 experts top-2): Q4_K / Q6_K 2048x5632 at 1.5, 3 and
-// 6 rows per expert 86 / 106, 125 / 104, 169 / 109; Q4_0 4096x14336 at 3, 4 and
-// 6 161 / 189, 208 / 205, 277 / 209.
+// decode / matrix cores, 8 experts top-2): Q4_K / Q6_K 2048x5632 at 1.5, 6, 8
+// and 16 rows per expert 53 / 105, 96 / 112, 113 / 113, 184 / 166; Q6_K
+// 4096x14336 at 6 and 8 365 / 451, 487 / 456; Q4_0 4096x14336 at 3, 4 and 6 161 /
+// 189, 208 / 205, 277 / 209.
 bool moe_q8_mfma_preferred(double rows_per_expert, bool q6, bool by_tile) {
     const char *e = std::getenv("RCE_QMM_Q8_MFMA");
     const int mode = e ? std::atoi(e) : 1;
     if (mode != 1) return mode == 2;
-    return !by_tile || rows_per_expert >= (q6 ? 2.5 : 4.0);
+    return !by_tile || rows_per_expert >= (q6 ? 8.0 : 4.0);
 }
 
 // The grouped experts: h = silu(W1 x) (w3 == nullptr, the benchmark's

@@ -600,7 +600,6 @@ static size_t unit_bytes(uint32_t dtype) {
     case T_STQ1_0: return 42;
     case T_Q4_K: return 36;
     case T_Q5_K: return 44;
-    case T_Q6_K: return 210;
     default: return 0;
     }
 }
@@ -608,9 +607,7 @@ static size_t unit_bytes(uint32_t dtype) {
 // Launch shape.  Measured on MI355X (the sweep over threads x rows per
 // thread x tokens per block): the best single-token shapes stream about
 // 36 KB of weight per 256-thread block with every load issued up front,
-// and keep at least one block per CU; Q6_K (one 210-byte super-block per
-// thread-row, heavy activation slice) is best at 4 rows per thread.  With
-// several tokens, Q8 keeps up to 8 per block (the weight tile is read once
+// and keep at least one block per CU.  With several tokens, Q8 keeps up to 8 per block (the weight tile is read once
 // per block) and EXACT 2, with 16 rows per lane where the grid keeps 256
 // blocks (below).
 GemvGeom pick_gemv_geom(const DevWeight &w, size_t t_rows, int mode) {
@@ -620,13 +617,11 @@ GemvGeom pick_gemv_geom(const DevWeight &w, size_t t_rows, int mode) {
     const bool q8 = mode == 1;
     const int P = g.nt / U;
     const bool k4 = w.dtype == T_Q4_K || w.dtype == T_Q5_K;  // 64-value units
-    int tbmax = q8 ? (w.dtype == T_Q6_K ? 2 : (k4 ? 4 : 8)) : (k4 ? 2 : 4);
-    if ((w.dtype == T_Q6_K && !q8) || is_ternary_block(w.dtype)) tbmax = 1;
+    int tbmax = q8 ? (k4 ? 4 : 8) : (k4 ? 2 : 4);
+    if (is_ternary_block(w.dtype)) tbmax = 1;
     g.tb = 1;
     while (g.tb * 2 <= tbmax && (size_t)g.tb * 2 <= t_rows) g.tb *= 2;
-    if (w.dtype == T_Q6_K) {
-        g.rpl = 4;
-    } else if (g.tb == 1 && !q8 && !is_ternary_block(w.dtype)) {
+    if (g.tb == 1 && !q8 && !is_ternary_block(w.dtype)) {
         // One token, EXACT (bound by its f32 arithmetic, so the work of the
         // busiest CU decides): the rows per lane that give the busiest of the 256 CUs
         // the least work, counted as blocks per CU x (rows per block + 8):
@@ -690,6 +685,7 @@ hipError_t launch_gemv(const DevWeight &w, const float *a, size_t t_rows, float 
     if (t_rows == 0 || w.n_rows == 0) return hipSuccess;
     if (mode != 0 && mode != 1) return hipErrorInvalidValue;
     if (is_row_chain(w.dtype)) return launch_gemv_chain(w, a, t_rows, out, s);
+    if (w.dtype == T_Q6_K) return launch_gemv_q6_k(w, a, t_rows, out, mode, s);
     const GemvGeom g = geom ? *geom : pick_gemv_geom(w, t_rows, is_ternary_block(w.dtype) ? 0 : mode);
     if (is_ternary_block(w.dtype)) return launch_gemv_ternary(w, g, a, t_rows, out, s);
     switch (w.dtype) {
@@ -697,7 +693,6 @@ hipError_t launch_gemv(const DevWeight &w, const float *a, size_t t_rows, float 
     case T_Q8_0: return launch_gemv_q8_0(w, g, a, t_rows, out, mode, s);
     case T_Q4_K: return launch_gemv_q4_k(w, g, a, t_rows, out, mode, s);
     case T_Q5_K: return launch_gemv_q5_k(w, g, a, t_rows, out, mode, s);
-    case T_Q6_K: return launch_gemv_q6_k(w, g, a, t_rows, out, mode, s);
     case T_Q5_0: return launch_gemv_q5_0(w, g, a, t_rows, out, mode, s);
     case T_Q4_1: return launch_gemv_q4_1(w, g, a, t_rows, out, mode, s);
     case T_Q3_K: return launch_gemv_q3_k(w, g, a, t_rows, out, mode, s);
@@ -722,6 +717,7 @@ hipError_t launch_gemv_fx(const FxLaunch &f, const float *a, int mode, hipStream
     if (!gemv_fx_supports(w.dtype, w.n_cols, mode, (f.kind & FX_NORM) != 0)) return hipErrorInvalidValue;
     for (int i = 1; i < f.nw; i++)
         if (f.w[i].dtype != w.dtype || f.w[i].n_cols != w.n_cols) return hipErrorInvalidValue;
+    if (w.dtype == T_Q6_K) return launch_gemv_fx_q6_k(f, a, mode, s);
     GemvGeom g = pick_gemv_geom(w, 1, mode);
     if (g.rpl > 8) g.rpl = 8;  // the fused forms exist for 1, 2, 4 and 8 rows per lane
     // Rows per lane, measured on the decode step's shapes (2048-11264 rows):
@@ -743,7 +739,6 @@ hipError_t launch_gemv_fx(const FxLaunch &f, const float *a, int mode, hipStream
     case T_Q8_0: return launch_gemv_fx_q8_0(f, g, a, mode, s);
     case T_Q4_K: return launch_gemv_fx_q4_k(f, g, a, mode, s);
     case T_Q5_K: return launch_gemv_fx_q5_k(f, g, a, mode, s);
-    case T_Q6_K: return launch_gemv_fx_q6_k(f, g, a, mode, s);
     case T_Q5_0: return launch_gemv_fx_q5_0(f, g, a, mode, s);
     case T_Q4_1: return launch_gemv_fx_q4_1(f, g, a, mode, s);
     case T_Q3_K: return launch_gemv_fx_q3_k(f, g, a, mode, s);
@@ -761,6 +756,7 @@ hipError_t launch_gemv_q8_pre(const DevWeight &w, const float *a, size_t t_rows,
                               hipStream_t s) {
     if (t_rows == 0 || w.n_rows == 0) return hipSuccess;
     if (!gemv_q8_pre_supports(w.dtype, w.n_cols, t_rows)) return launch_gemv(w, a, t_rows, out, 1, s);
+    if (w.dtype == T_Q6_K) return launch_gemv(w, a, t_rows, out, 1, s);  // its blocks quantize their two tokens
     GemvGeom g = pick_gemv_geom(w, t_rows, 1);
     if (g.nt != 256 || g.tb < 2) return launch_gemv(w, a, t_rows, out, 1, s);
     if (g.tb > 4) g.tb = 4;  // more token groups re-read the weight, mostly from the Infinity Cache
@@ -785,7 +781,6 @@ hipError_t launch_gemv_q8_pre(const DevWeight &w, const float *a, size_t t_rows,
     case T_Q8_0: return launch_as_preq_tb<Q8_0Q8, 8>(w, g, a, t_rows, out, q, s);
     case T_Q4_K: return launch_as_preq_tb<Q4_KQ8, 4>(w, g, a, t_rows, out, q, s);
     case T_Q5_K: return launch_as_preq_tb<Q5_KQ8, 4>(w, g, a, t_rows, out, q, s);
-    case T_Q6_K: return launch_as_preq_tb<Q6_KQ8, 2>(w, g, a, t_rows, out, q, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -822,9 +817,7 @@ bool gemv_grouped_supports(uint32_t dtype, size_t n_cols, int mode) {
     if (!gpu_supports(dtype, n_cols, mode)) return false;
     switch (dtype) {
     case T_Q4_0: case T_Q8_0: case T_Q5_0: case T_Q4_1: case T_Q3_K: case T_Q4_K: case T_Q5_K: break;
-    case T_Q6_K:
-        if (mode == 0) return n_cols <= 16384;
-        break;
+    case T_Q6_K: return mode != 0 || n_cols <= 16384;
     default: return false;
     }
     const int U = units_per_row(dtype, n_cols), nt = nt_for(U);

@@ -1199,80 +1199,6 @@ struct Q5_KQ8 {
     }
 };
 
-// Q6_K super-block, Q8: for sub-blocks b of 16 ascending,
-// ssb += (d sc_b) (dx isum_b) from +0.0; the addend is ssb.
-template <int TB>
-struct Q6_KQ8 {
-    static constexpr int NTOK = TB;
-    using Raw = RawQ6_K;
-    int xw[TB][64];
-    float dx[TB][8];
-    int s16[TB][16];
-    __device__ static Raw load(const DevWeight &w, size_t row, int col) {
-        Raw r;
-        ld_q6_k(w, row, col, r);
-        return r;
-    }
-    __device__ void init_q8(const ActLds &L, size_t k, int tv, int col) {
-#pragma unroll
-        for (int t = 0; t < TB; t++) {
-            const bool ok = t < tv;
-            const size_t tt = ok ? (size_t)t : 0;
-            const int4 *p = reinterpret_cast<const int4 *>(L.xq + (tt * k + 256 * (size_t)col) / 4);
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int4 v = p[i];
-                xw[t][4 * i] = ok ? v.x : 0; xw[t][4 * i + 1] = ok ? v.y : 0;
-                xw[t][4 * i + 2] = ok ? v.z : 0; xw[t][4 * i + 3] = ok ? v.w : 0;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i++) dx[t][i] = ok ? L.dx[tt * (k / 32) + 8 * (size_t)col + i] : 0.0f;
-#pragma unroll
-            for (int i = 0; i < 16; i++) s16[t][i] = ok ? L.s16[tt * (k / 16) + 16 * (size_t)col + i] : 0;
-        }
-    }
-    __device__ void addends(const Raw &b, float *out) const {
-        const float d = h2f(b.d);
-        float ssb[TB];
-#pragma unroll
-        for (int t = 0; t < TB; t++) ssb[t] = 0.0f;
-#pragma unroll
-        for (int o = 0; o < 2; o++) {
-            int acc[TB][8];  // sub-block 8o + 2m + c -> index 2m + c
-#pragma unroll
-            for (int t = 0; t < TB; t++)
-#pragma unroll
-                for (int i = 0; i < 8; i++) acc[t][i] = 0;
-#pragma unroll
-            for (int lq = 0; lq < 8; lq++) {
-                uint32_t u[4];
-                q6_words(b, o, lq, u[0], u[1], u[2], u[3]);
-                const int c = lq >> 2, wi = lq & 3;
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-#pragma unroll
-                    for (int t = 0; t < TB; t++)
-                        acc[t][2 * m + c] = __builtin_amdgcn_sdot4((int)u[m], xw[t][32 * o + 8 * m + 4 * c + wi],
-                                                                   acc[t][2 * m + c], false);
-                }
-            }
-#pragma unroll
-            for (int bb = 0; bb < 8; bb++) {
-                const int sbk = 8 * o + bb;
-                const float ds = d * (float)q6_sc(b.c[12], sbk);
-#pragma unroll
-                for (int t = 0; t < TB; t++) {
-                    const int isum = acc[t][bb] - 32 * s16[t][sbk];
-                    const float ab = dx[t][sbk >> 1] * (float)isum;
-                    ssb[t] = ssb[t] + ds * ab;
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TB; t++) out[t] = ssb[t];
-    }
-};
-
 // ---------------------------------------------------------------------------
 // The activation-stationary kernel.
 // ---------------------------------------------------------------------------
@@ -1284,7 +1210,7 @@ __host__ __device__ constexpr int fold_ld(int U) { return ((U + 3) & ~3) + 4; }
 template <class U, class = void> struct HasPrepare : std::false_type {};
 template <class U> struct HasPrepare<U, std::void_t<decltype(std::declval<U &>().prepare())>> : std::true_type {};
 // Units whose weights load through a WBuf (every layout with whole rows at
-// row_stride; LAYOUT_IL64_Q6_K interleaves 64 rows and keeps the pointer form).
+// row_stride).
 template <class U, class = void> struct HasLoadB : std::false_type {};
 template <class U>
 struct HasLoadB<U, std::void_t<decltype(U::load_b(std::declval<const DevWeight &>(), std::declval<const WBuf &>(),

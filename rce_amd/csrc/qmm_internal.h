@@ -253,7 +253,7 @@ hipError_t launch_gemv_fx_q4_0(const FxLaunch &f, const GemvGeom &g, const float
 hipError_t launch_gemv_fx_q8_0(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
 hipError_t launch_gemv_fx_q4_k(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
 hipError_t launch_gemv_fx_q5_k(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
-hipError_t launch_gemv_fx_q6_k(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
+hipError_t launch_gemv_fx_q6_k(const FxLaunch &f, const float *a, int mode, hipStream_t s);
 hipError_t launch_gemv_fx_q5_0(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
 hipError_t launch_gemv_fx_q4_1(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
 hipError_t launch_gemv_fx_q3_k(const FxLaunch &f, const GemvGeom &g, const float *a, int mode, hipStream_t s);
@@ -346,7 +346,7 @@ hipError_t launch_gemv_q4_k(const DevWeight &w, const GemvGeom &g, const float *
                             int mode, hipStream_t s);
 hipError_t launch_gemv_q5_k(const DevWeight &w, const GemvGeom &g, const float *a, size_t t_rows, float *out,
                             int mode, hipStream_t s);
-hipError_t launch_gemv_q6_k(const DevWeight &w, const GemvGeom &g, const float *a, size_t t_rows, float *out,
+hipError_t launch_gemv_q6_k(const DevWeight &w, const float *a, size_t t_rows, float *out,
                             int mode, hipStream_t s);
 hipError_t launch_gemv_q5_0(const DevWeight &w, const GemvGeom &g, const float *a, size_t t_rows, float *out,
                             int mode, hipStream_t s);
