@@ -5,6 +5,10 @@
 // fragments in registers and contracted with v_mfma_f32_32x32x16_f16 (f32
 // accumulation).
 //
+// Short M (gemm_slices): K in slices of whole scale groups, one grid row
+// each, where the tiles alone leave CUs idle; the slices' sums are added in
+// order by a second kernel.
+//
 // Tiling.  A block owns a BM x BN (M x N) output tile: 128 x 64 or 64 x 128
 // (8192 outputs), so a 512 x 4096 product is 256 tiles, one per CU; or
 // 96 x 128 for the grouped mode when experts get about 64 rows each (65-96
@@ -73,6 +77,7 @@
 #include "mfma_util.h"
 #include "qmm_internal.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace rce_qmm {
@@ -319,12 +324,13 @@ struct Q6K {
 template <class T, class Fmt, int EPI>
 __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__restrict__ A, uint32_t a_bytes,
                                           void *__restrict__ out_v, const float *__restrict__ aux, size_t m0,
-                                          int rows, size_t n0, const int *arow, unsigned char *lds) {
+                                          int rows, size_t n0, const int *arow, unsigned char *lds, int gb = 0, int slice_groups = 0, bool add = false) {
     constexpr int BM = T::BM, BN = T::BN, RB = T::RB, CB = T::CB, NS = T::NS, NH = Fmt::NH;
     constexpr int A_STAGE = T::A_STAGE, W_HALF = T::W_HALF, W_GROUP = T::W_GROUP;
     constexpr int OFF_W = T::OFF_W;
     const size_t N = w.n_rows, K = w.n_cols;
-    const int nchunks = (int)(K / KC), ngroups = nchunks / 4;
+    constexpr bool SLICE = EPI == GEPI_SLICE;  // only scale groups gb .. gb + slice_groups - 1
+    const int nchunks = SLICE ? 4 * slice_groups : (int)(K / KC), ngroups = nchunks / 4;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool producer = wave >= NC / 64;
@@ -395,7 +401,7 @@ __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__
         const __amdgpu_buffer_rsrc_t wbuf =
             Fmt::IL64 ? byte_buffer(w.base + (n0 >> 6) * w.group_stride, (uint32_t)w.group_stride)
                       : byte_buffer(w.base + n0 * w.row_stride, (uint32_t)(wtile * w.row_stride));
-        const uint32_t a_soff_max = (uint32_t)(nchunks - 1) * (KC * 2);
+        const uint32_t a_soff0 = SLICE ? (uint32_t)gb * (4 * KC * 2) : 0, a_soff_max = a_soff0 + (uint32_t)(nchunks - 1) * (KC * 2);
         // W position q of group gs into the group buffer dst: at 0 the
         // weight bytes (split formats: the 64-byte pieces pw, pw + 2, ... of
         // every row; IL64: chunks 6 pw .. 6 pw + 5), at 1 the headers of
@@ -446,9 +452,9 @@ __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__
             const int q = it & 3;
             if (q < 2) {
                 const int g = (it >> 2) + GA, gs = g < ngroups ? g : ngroups - 1;
-                load_w(q, gs, lds + OFF_W + (g & (NWBUF - 1)) * W_GROUP);
+                load_w(q, SLICE ? gb + gs : gs, lds + OFF_W + (g & (NWBUF - 1)) * W_GROUP);
             }
-            const uint32_t soff = __builtin_elementwise_min((uint32_t)(it + NS - 1) * (KC * 2), a_soff_max);
+            const uint32_t soff = __builtin_elementwise_min(a_soff0 + (uint32_t)(it + NS - 1) * (KC * 2), a_soff_max);
             unsigned char *dst = lds + ((it + NS - 1) % NS) * A_STAGE + pw * (A_STAGE / 2);
 #pragma unroll
             for (int i = 0; i < T::A_LOADS; i++) buf_load_lds16(abuf, a_lane[i], soff, dst + i * 1024);
@@ -458,10 +464,10 @@ __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__
         for (int it = -4 * GA; it < 0; it++) {
             if ((it & 3) < 2) {
                 const int q = it & 3, g = (it >> 2) + GA, gs = g < ngroups ? g : ngroups - 1;
-                load_w(q, gs, lds + OFF_W + (g & (NWBUF - 1)) * W_GROUP);
+                load_w(q, SLICE ? gb + gs : gs, lds + OFF_W + (g & (NWBUF - 1)) * W_GROUP);
             }
             if (it + NS - 1 >= 0) {
-                const uint32_t soff = __builtin_elementwise_min((uint32_t)(it + NS - 1) * (KC * 2), a_soff_max);
+                const uint32_t soff = __builtin_elementwise_min(a_soff0 + (uint32_t)(it + NS - 1) * (KC * 2), a_soff_max);
                 unsigned char *dst = lds + ((it + NS - 1) % NS) * A_STAGE + pw * (A_STAGE / 2);
 #pragma unroll
                 for (int i = 0; i < T::A_LOADS; i++) buf_load_lds16(abuf, a_lane[i], soff, dst + i * 1024);
@@ -699,6 +705,9 @@ __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__
                         const size_t o = (m0 + m) * N + col;
                         if constexpr (EPI == GEPI_F32) {
                             static_cast<float *>(out_v)[o] = sum[e];
+                        } else if constexpr (EPI == GEPI_SLICE) {
+                            float *op = static_cast<float *>(out_v) + o;
+                            *op = add ? *op + sum[e] : sum[e];
                         } else if constexpr (EPI == GEPI_SILU_F16) {  // rce-qwen36-moe/src/lib.rs L459-461
                             static_cast<_Float16 *>(out_v)[o] = (_Float16)silu_mfma(sum[e]);
                         } else {  // silu(g) * u, rce-qwen36-moe/src/lib.rs L667-676
@@ -720,7 +729,7 @@ __global__ __launch_bounds__(NT) void k_gemm_f16(DevWeight w_arg, const _Float16
                                                  const int *__restrict__ gather, size_t M, uint32_t a_bytes,
                                                  void *__restrict__ out_v, const float *__restrict__ aux, int m_tiles,
                                                  const MoeTile *__restrict__ tiles, const int *__restrict__ n_tiles,
-                                                 const DevWeight *__restrict__ wtab) {
+                                                 const DevWeight *__restrict__ wtab, int slice0, int slices) {
     using T = Tile<BM_, Fmt, BN_>;
     constexpr int BM = T::BM;
     extern __shared__ __align__(16) unsigned char lds[];
@@ -760,6 +769,16 @@ __global__ __launch_bounds__(NT) void k_gemm_f16(DevWeight w_arg, const _Float16
     }
     __syncthreads();
     const size_t n0 = (size_t)nt * T::BN;
+    // GEPI_SLICE: this block's K slice is slice0 + blockIdx.y of `slices`.  A
+    // launch of several writes slice y's sums to rows y M .. of out_v; one of
+    // a single later slice adds to out_v.
+    if constexpr (EPI == GEPI_SLICE) {
+        const int groups = (int)(w.n_cols / (4 * KC)), slice = slice0 + (int)blockIdx.y;
+        const int gb = groups * slice / slices, ng = groups * (slice + 1) / slices - gb;
+        gemm_tile<T, Fmt, EPI>(w, A, a_bytes, out_v, aux, m0 + blockIdx.y * M, rows, n0, arow, lds, gb, ng,
+                               gridDim.y == 1 && slice > 0);
+        return;
+    }
     // A 96- or 128-row tile that holds at most 64 rows (a grouped tile whose
     // expert has that few, a plain GEMM's last row tile) runs the 64-row
     // tile's body over the same columns: a third or half fewer activation
@@ -791,20 +810,44 @@ __global__ void k_f32_to_f16(const float *__restrict__ s, _Float16 *__restrict__
     if (i < n) d[i] = (_Float16)s[i];
 }
 
+// Eight values per thread (two 16-byte loads, one 16-byte store), against one:
+// 77 x 5632 values 3.3 -> 2.1 us, 4096 x 4096 25 -> 15 (6.7 TB/s), 4096 x 14336
+// 130 -> 58.
+__global__ __launch_bounds__(256) void k_f32_to_f16_x8(const float4 *__restrict__ s, half8 *__restrict__ d, size_t n8) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const float4 a = s[2 * i], b = s[2 * i + 1];
+    d[i] = half8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
+                 (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
+}
+
+// out[i] = the K slices' sums added in slice order (deterministic).
+template <class V>
+__global__ __launch_bounds__(256) void k_sum_slices(const V *__restrict__ parts, V *__restrict__ out, size_t n, int slices) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    V v = parts[i];
+#pragma unroll 4
+    for (int y = 1; y < slices; y++) v += parts[i + (size_t)y * n];
+    out[i] = v;
+}
+
 template <class Fmt, int BM, int EPI, int BN_ = 0>
 hipError_t set_lds_attr() {
     return ensure_lds_limit((const void *)k_gemm_f16<Fmt, BM, EPI, BN_>, Tile<BM, Fmt, BN_>::LDS);
 }
 
-template <class Fmt, int BM, int BN_ = 0>
-hipError_t launch_fmt(const DevWeight &w, const _Float16 *a, size_t M, float *out, hipStream_t s) {
+// K slices slice0 .. slice0 + count - 1 of `slices` (EPI GEPI_SLICE), or all of K.
+template <class Fmt, int BM, int BN_ = 0, int EPI = GEPI_F32>
+hipError_t launch_fmt(const DevWeight &w, const _Float16 *a, size_t M, float *out, hipStream_t s, int slice0 = 0,
+                      int count = 1, int slices = 1) {
     using T = Tile<BM, Fmt, BN_>;
     const int m_tiles = (int)((M + T::BM - 1) / T::BM), n_tiles = (int)((w.n_rows + T::BN - 1) / T::BN);
-    hipError_t e = set_lds_attr<Fmt, BM, GEPI_F32, BN_>();
+    hipError_t e = set_lds_attr<Fmt, BM, EPI, BN_>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_gemm_f16<Fmt, BM, GEPI_F32, BN_>), dim3(m_tiles * n_tiles), dim3(NT), T::LDS, s, w, a,
+    hipLaunchKernelGGL((k_gemm_f16<Fmt, BM, EPI, BN_>), dim3(m_tiles * n_tiles, count), dim3(NT), T::LDS, s, w, a,
                        (const int *)nullptr, M, (uint32_t)(M * w.n_cols * 2), (void *)out, (const float *)nullptr,
-                       m_tiles, (const MoeTile *)nullptr, (const int *)nullptr, (const DevWeight *)nullptr);
+                       m_tiles, (const MoeTile *)nullptr, (const int *)nullptr, (const DevWeight *)nullptr, slice0, slices);
     return hipGetLastError();
 }
 
@@ -817,7 +860,8 @@ hipError_t launch_fmt_grouped(const DevWeight &w, const DevWeight *wtab, const _
     hipError_t e = set_lds_attr<Fmt, BM, EPI>();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_gemm_f16<Fmt, BM, EPI>), dim3(grouped_grid(max_tiles, n_tiles)), dim3(NT), T::LDS, s, w, a,
-                       gather, a_rows, (uint32_t)(a_rows * w.n_cols * 2), out, aux, max_tiles, tiles, n_tiles_dev, wtab);
+                       gather, a_rows, (uint32_t)(a_rows * w.n_cols * 2), out, aux, max_tiles, tiles, n_tiles_dev, wtab, 0,
+                       1);
     return hipGetLastError();
 }
 
@@ -866,6 +910,7 @@ hipError_t gemm_prepare_lds() {
         all_epi(fmt, ic<128>{});
         // the plain GEMM's 64 x 64 tile (short M)
         if (e == hipSuccess) e = set_lds_attr<F, 64, GEPI_F32, 64>();
+        if (e == hipSuccess) e = set_lds_attr<F, 64, GEPI_SLICE, 64>();
     };
     all_bm(Q4K{});
     all_bm(Q5K{});
@@ -876,6 +921,8 @@ hipError_t gemm_prepare_lds() {
     all_epi(Q6K{}, ic<128>{});
     if (e == hipSuccess) e = set_lds_attr<Q80, 64, GEPI_F32, 64>();
     if (e == hipSuccess) e = set_lds_attr<Q6K, 64, GEPI_F32, 64>();
+    if (e == hipSuccess) e = set_lds_attr<Q80, 64, GEPI_SLICE, 64>();
+    if (e == hipSuccess) e = set_lds_attr<Q6K, 64, GEPI_SLICE, 64>();
     return e;
 }
 
@@ -892,8 +939,12 @@ bool gemm_supports(uint32_t dtype, size_t n_cols) {
 
 hipError_t launch_f32_to_f16(const float *src, void *dst, size_t n, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_f32_to_f16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, src,
-                       static_cast<_Float16 *>(dst), n);
+    if (n % 8 == 0 && (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) % 16 == 0 && n / 8 <= ((size_t)1 << 31))
+        hipLaunchKernelGGL(k_f32_to_f16_x8, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s,
+                           reinterpret_cast<const float4 *>(src), static_cast<half8 *>(dst), n / 8);
+    else
+        hipLaunchKernelGGL(k_f32_to_f16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, src,
+                           static_cast<_Float16 *>(dst), n);
     return hipGetLastError();
 }
 
@@ -954,17 +1005,23 @@ int cu_count() {
     return c > 0 ? c : 0;
 }
 
-hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, int bm) {
-    if (M == 0 || w.n_rows == 0) return hipSuccess;
-    if (!gemm_shape_ok(M, w)) return hipErrorInvalidValue;
-    const _Float16 *a = static_cast<const _Float16 *>(a_f16);
-    const size_t n64 = (w.n_rows + 63) / 64, m64 = (M + 63) / 64, cus = cu_count() ? (size_t)cu_count() : 256;
+namespace {
+
+// The plain GEMM's launch: row tile bm (0: the rule's), or the 64 x 64 tile.
+struct GemmTile {
+    int bm;
+    bool sq64;
+    size_t tiles;
+};
+
+GemmTile pick_gemm_tile(const DevWeight &w, size_t M, size_t cus, int bm) {
+    const size_t n64 = (w.n_rows + 63) / 64, m64 = (M + 63) / 64;
     // Q8_0 / Q6_K: 64-column tiles only, 128 rows, or 64 where that makes
     // more blocks in one round (below)
     if (gemm_q8_supports(w.dtype, w.n_cols)) {
-        const bool q64 = bm == 0 && ((M + 127) / 128) * n64 < cus && m64 * n64 <= cus;
-        if (w.dtype == T_Q8_0) return q64 ? launch_fmt<Q80, 64, 64>(w, a, M, out, s) : launch_fmt<Q80, 128>(w, a, M, out, s);
-        return q64 ? launch_fmt<Q6K, 64, 64>(w, a, M, out, s) : launch_fmt<Q6K, 128>(w, a, M, out, s);
+        const size_t t128 = ((M + 127) / 128) * n64;
+        const bool q64 = bm == 0 && t128 < cus && m64 * n64 <= cus;
+        return {q64 ? 64 : 128, q64, q64 ? m64 * n64 : t128};
     }
     bool sq64 = false;  // the 64 x 64 tile
     if (bm == 0) {
@@ -988,19 +1045,79 @@ hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, floa
         const size_t bn = bm == 128 ? 64 : 128;
         sq64 = ((M + bm - 1) / bm) * ((w.n_rows + bn - 1) / bn) < cus && m64 * n64 <= cus;
     }
-    hipError_t e = hipErrorInvalidValue;
-    with_fmt(w.dtype, [&](auto fmt) {
+    const size_t bn = bm == 128 ? 64 : 128;
+    return {bm, sq64, sq64 ? m64 * n64 : ((M + bm - 1) / bm) * ((w.n_rows + bn - 1) / bn)};
+}
+
+// K slices of a plain GEMM whose tiles leave CUs idle (short M): as many as
+// there are CUs for, if the time they save is more than their sums cost.
+// Estimated from Q4_K and Q6_K at M 16-256, N 512-8192, K 1024-14336 (us): a
+// tile takes 4.4 + 0.56 per scale group (256 of K), the slices' sums 3 (the
+// second launch) + 0.6 per MB of them.  Measured there, one piece / sliced:
+// Q6_K 2048x5632 at M 16 19.3 / 10.0 (6), at 77 19.6 / 12.5 (4), at 256 19.7 /
+// 16.7 (2); 4096x14336 at 16 41.8 / 17.9 (4), at 128 42.4 / 30.3 (2); Q4_K
+// 4096x4096 at 16 13.4 / 10.3 (4), at 128 13.9 / 13.9 (2: not taken); 2048x2048
+// at 77 9.4 / 9.7 (4: not taken).  The result depends on the slice count alone.
+int gemm_slices(const DevWeight &w, size_t M, const GemmTile &t, size_t cus) {
+    if (!t.sq64) return 1;  // the sliced form exists for the 64 x 64 tile, the one a chip with idle CUs runs
+    const int groups = (int)std::min<size_t>(w.n_cols / (4 * KC), 1 << 20), most = (int)std::min({cus / t.tiles, (size_t)groups, (size_t)16});
+    const double mb = (double)M * (double)w.n_rows * 4e-6, whole = 0.56 * groups;
+    int best = 1;
+    double cost = whole - 0.5;
+    for (int n = 2; n <= most; n++) {
+        const double c = 0.56 * ((groups + n - 1) / n) + 3.0 + 0.6 * mb * n;
+        if (c < cost) { cost = c; best = n; }
+    }
+    return best;
+}
+
+}  // namespace
+
+size_t gemm_f16_slice_bytes(const DevWeight &w, size_t M) {
+    if (M == 0 || w.n_rows == 0 || !gemm_shape_ok(M, w) || !(gemm_supports(w.dtype, w.n_cols) || gemm_q8_supports(w.dtype, w.n_cols)))
+        return 0;
+    const size_t cus = cu_count() ? (size_t)cu_count() : 256;
+    const int sl = gemm_slices(w, M, pick_gemm_tile(w, M, cus, 0), cus);
+    return sl == 1 ? 0 : (size_t)sl * M * w.n_rows * sizeof(float);
+}
+
+hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, int bm, float *parts) {
+    if (M == 0 || w.n_rows == 0) return hipSuccess;
+    if (!gemm_shape_ok(M, w)) return hipErrorInvalidValue;
+    const _Float16 *a = static_cast<const _Float16 *>(a_f16);
+    const size_t cus = cu_count() ? (size_t)cu_count() : 256;
+    const GemmTile g = pick_gemm_tile(w, M, cus, bm);
+    const int sl = bm == 0 ? gemm_slices(w, M, g, cus) : 1;
+    // without room for the slices' sums: slice after slice, each adding to
+    // the output (the same bits)
+    float *o = sl > 1 && parts ? parts : out;
+    const int count = sl > 1 && parts ? sl : 1;
+    hipError_t e = hipSuccess;
+    auto launch = [&](auto fmt, auto q8_layout) {
         using F = decltype(fmt);
-        if (sq64)
-            e = launch_fmt<F, 64, 64>(w, a, M, out, s);
-        else if (bm == 64)
-            e = launch_fmt<F, 64>(w, a, M, out, s);
-        else if (bm == 96)
-            e = launch_fmt<F, 96>(w, a, M, out, s);
-        else if (bm == 128)
-            e = launch_fmt<F, 128>(w, a, M, out, s);
-    });
-    return e;
+        if (sl > 1) {  // 64 x 64 tiles
+            for (int y = 0; y < sl && e == hipSuccess; y += count) e = launch_fmt<F, 64, 64, GEPI_SLICE>(w, a, M, o, s, y, count, sl);
+        } else if (g.sq64) {
+            e = launch_fmt<F, 64, 64>(w, a, M, o, s);
+        } else if (g.bm == 128) {
+            e = launch_fmt<F, 128>(w, a, M, o, s);
+        } else if constexpr (decltype(q8_layout)::value) {
+            e = hipErrorInvalidValue;
+        } else {
+            e = g.bm == 64 ? launch_fmt<F, 64>(w, a, M, o, s) : (g.bm == 96 ? launch_fmt<F, 96>(w, a, M, o, s) : hipErrorInvalidValue);
+        }
+    };
+    if (w.dtype == T_Q8_0) launch(Q80{}, ic<1>{});
+    else if (w.dtype == T_Q6_K) launch(Q6K{}, ic<1>{});
+    else if (!with_fmt(w.dtype, [&](auto fmt) { launch(fmt, ic<0>{}); })) e = hipErrorInvalidValue;
+    if (e != hipSuccess || count == 1) return e;
+    const size_t n = M * w.n_rows;
+    if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(parts)) % 16 == 0)
+        hipLaunchKernelGGL(k_sum_slices<f32x4>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
+                           reinterpret_cast<const f32x4 *>(parts), reinterpret_cast<f32x4 *>(out), n / 4, sl);
+    else
+        hipLaunchKernelGGL(k_sum_slices<float>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const float *)parts, out, n, sl);
+    return hipGetLastError();
 }
 
 }  // namespace rce_qmm

@@ -68,6 +68,7 @@ struct BatchedScratch {
     float *a_f32 = nullptr;       // F16 activations widened to f32 (EXACT, Q8)
     unsigned char *act_q = nullptr;  // Q8 activations of several tokens, quantized once
     void *a_f16 = nullptr;        // F32 activations rounded to f16 (F16_MFMA)
+    float *parts = nullptr;       // the sums of the GEMM's K slices (F16_MFMA, short M)
 };
 
 }  // namespace
@@ -103,15 +104,15 @@ rce_qmm_status run_gemm(const void *a_dev, bool a_f16, size_t t_rows, const DevW
     }
     if (gemm_supports(dw.dtype, dw.n_cols) || gemm_q8_supports(dw.dtype, dw.n_cols)) {
         // The kernel's activation offsets are 32-bit: slices of whole
-        // 128-row tiles below 2^32 bytes each (each output's sum does not
-        // depend on the slicing).
+        // 128-row tiles below 2^32 bytes each (an output's sum depends on the
+        // slicing only through the K slices of a short last slice).
         const size_t k = dw.n_cols, max_rows = ((((size_t)1 << 32) - 1) / (k * 2)) / 128 * 128;
         if (max_rows == 0)
             return fail(RCE_QMM_BAD_SHAPE, "n_cols " + std::to_string(k) + " is too long for the F16_MFMA GEMM");
         const _Float16 *a16 = static_cast<const _Float16 *>(a);
         for (size_t r0 = 0; r0 < t_rows; r0 += max_rows) {
             const size_t rows = t_rows - r0 < max_rows ? t_rows - r0 : max_rows;
-            HIP_TRY(launch_gemm_f16(dw, a16 + r0 * k, rows, out_dev + r0 * dw.n_rows, s));
+            HIP_TRY(launch_gemm_f16(dw, a16 + r0 * k, rows, out_dev + r0 * dw.n_rows, s, 0, rows == t_rows ? sc.parts : nullptr));
         }
     } else {
         HIP_TRY(launch_gemm_gen(dw, a, t_rows, out_dev, s));
@@ -152,6 +153,14 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
         else q8_b = b;
     }
     const size_t f16_b = mfma && a_dtype == T_F32 ? t_rows * k * 2 : 0;
+    // The GEMM's K slices: without room for their sums (the fixed scratch; a
+    // buffer to grow under stream capture) they run one after another.
+    size_t part_b = mfma && !gemm_wide_preferred(dw, t_rows) ? gemm_f16_slice_bytes(dw, t_rows) : 0;
+    if (part_b && fixed && align_up(f16_b, 256) + align_up(part_b, 256) > fixed_cap) part_b = 0;
+    if (part_b && !fixed && ctx->parts.cap < part_b) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) part_b = 0;
+    }
     BatchedScratch sc;
     rce_qmm_status st;
     if (fixed) {
@@ -163,6 +172,7 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
         if (f32_b) { sc.a_f32 = reinterpret_cast<float *>(p); p += align_up(f32_b, 256); }
         if (q8_b) { sc.act_q = p; p += align_up(q8_b, 256); }
         if (f16_b) { sc.a_f16 = p; p += align_up(f16_b, 256); }
+        if (part_b) { sc.parts = reinterpret_cast<float *>(p); p += align_up(part_b, 256); }
     } else {
         if (f32_b) {
             if ((st = ensure(ctx, ctx->a_f32, f32_b, s))) return st;
@@ -175,6 +185,10 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
         if (f16_b) {
             if ((st = ensure(ctx, ctx->a_f16, f16_b, s))) return st;
             sc.a_f16 = ctx->a_f16.p;
+        }
+        if (part_b) {
+            if ((st = ensure(ctx, ctx->parts, part_b, s))) return st;
+            sc.parts = static_cast<float *>(ctx->parts.p);
         }
     }
     if (mfma) return run_gemm(a_dev, a_dtype == T_F16, t_rows, dw, out_dev, sc, s);
@@ -331,7 +345,7 @@ void rce_qmm_abi::context_release(rce_qmm_context *ctx) {
     if (ctx->refs.fetch_sub(1) != 1) return;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    for (Scratch *s : {&ctx->a_in, &ctx->a_f32, &ctx->out, &ctx->a_f16, &ctx->act_q, &ctx->moe_meta, &ctx->moe_wtab, &ctx->moe_x,
+    for (Scratch *s : {&ctx->a_in, &ctx->a_f32, &ctx->out, &ctx->a_f16, &ctx->parts, &ctx->act_q, &ctx->moe_meta, &ctx->moe_wtab, &ctx->moe_x,
                        &ctx->moe_h, &ctx->moe_h16, &ctx->moe_y, &ctx->moe_u})
         if (s->p) (void)hipFree(s->p);
     if (ctx->moe_grouped) (void)hipEventDestroy(ctx->moe_grouped);

@@ -380,7 +380,12 @@ bool gemm_q8_supports(uint32_t dtype, size_t n_cols);
 bool gemm_shape_ok(size_t a_rows, const DevWeight &w);
 // bm: output tile rows, 64 (tile 64 x 128), 96 (96 x 128) or 128 (128 x 64);
 // 0 = by M.
-hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, int bm = 0);
+// parts: gemm_f16_slice_bytes(w, M) bytes for the sums of K slices (null: the
+// slices run one after another, with the same bits).
+hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, int bm = 0,
+                           float *parts = nullptr);
+// The bytes launch_gemm_f16 would use for K slices (0: it uses none).
+size_t gemm_f16_slice_bytes(const DevWeight &w, size_t M);
 // The other formats' prefill GEMM (gemm_gen.hip): Q8_0, Q5_0, Q4_1, F16 (K
 // a multiple of 64), Q5_K, Q6_K (K a multiple of 256); nibble_forms also
 // admits Q4_0 and Q4_K (the same generic form, for cross-checks).  A must
@@ -500,7 +505,8 @@ hipError_t launch_moe_combine(const float *y, const int *slot_of_pair, const flo
 // What the grouped GEMM stores for output element o with f32 sum v:
 // v (f32 out), binary16 silu(v), or binary16 silu(aux[o]) * v (aux: the
 // f32 gate products of the same slots, SwiGLU).
-enum GemmEpilogue { GEPI_F32 = 0, GEPI_SILU_F16 = 1, GEPI_SWIGLU_F16 = 2 };
+// (GEPI_SLICE: f32 sums of a K slice, plain launches only)
+enum GemmEpilogue { GEPI_F32 = 0, GEPI_SILU_F16 = 1, GEPI_SWIGLU_F16 = 2, GEPI_SLICE = 3 };
 // Grouped GEMM: for every tile (expert e, slots r0 ..): out[r0 + m, :] =
 // epi(A[gather ? gather[r0 + m] : r0 + m, :] . wtab[e]^T).  `w` gives the
 // dtype and shape shared by all experts; wtab is a device array of
