@@ -1,4 +1,5 @@
-// gemv_q6_k.hip -- the Q6_K decode kernels (EXACT: one chain lane per row; Q8).
+// gemv_q6_k.hip -- the Q6_K decode kernels (EXACT: one chain lane per row; Q8: one
+// lane per row and super-block).
 #include "gemv_chain_pipe.h"
 #include "lds_limit.h"
 #include "qmm_gemv_kernels.h"

@@ -159,7 +159,12 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     if (part_b && fixed && align_up(f16_b, 256) + align_up(part_b, 256) > fixed_cap) part_b = 0;
     if (part_b && !fixed && ctx->parts.cap < part_b) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) part_b = 0;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            part_b = 0;
+        } else if (cap != hipStreamCaptureStatusNone) {
+            part_b = 0;
+        }
     }
     BatchedScratch sc;
     rce_qmm_status st;

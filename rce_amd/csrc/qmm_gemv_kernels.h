@@ -3,8 +3,8 @@
 // the Q8-activation GEMV (Q8), and row dequantization.
 //
 // Work mapping ("activation-stationary").  A row of the weight is U column
-// units (a Q4_0 / Q8_0 block of 32, a Q4_K group of 64, a Q6_K super-block
-// of 256).  Thread `tid` of a block of NT threads owns unit col = tid % U
+// units (a Q4_0 / Q8_0 block of 32, a Q4_K group of 64; Q6_K has kernels of
+// its own, gemv_q6_k.hip).  Thread `tid` of a block of NT threads owns unit col = tid % U
 // and the rows rsub, rsub + P, ... (rsub = tid / U, P = NT / U) of the
 // block's tile of RT = P * RPL rows, for TB activation rows (tokens).  It
 // keeps its slice of the activations in registers, issues the loads of all

@@ -507,11 +507,6 @@ hipError_t launch_moe_combine(const float *y, const int *slot_of_pair, const flo
 // f32 gate products of the same slots, SwiGLU).
 // (GEPI_SLICE: f32 sums of a K slice, plain launches only)
 enum GemmEpilogue { GEPI_F32 = 0, GEPI_SILU_F16 = 1, GEPI_SWIGLU_F16 = 2, GEPI_SLICE = 3 };
-// Grouped GEMM: for every tile (expert e, slots r0 ..): out[r0 + m, :] =
-// epi(A[gather ? gather[r0 + m] : r0 + m, :] . wtab[e]^T).  `w` gives the
-// dtype and shape shared by all experts; wtab is a device array of
-// DevWeight; a_rows: rows of A (bounds the loads); max_tiles bounds
-// n_tiles_dev[0].
 // The Q8 mode of grouped experts on the int8 matrix cores (gemv_q8_mfma.hip):
 // tiles of 16 slots.  launch_quantize_tiles fills `acts`
 // (gemv_q8_tile_bytes(k) per tile) from the rows of a: src Q8SRC_ROWS the
@@ -524,6 +519,11 @@ hipError_t launch_quantize_tiles(int src, const float *a, const float *a2, size_
                                  const MoeTile *tiles, const int *n_tiles, const int *tok_of_slot, void *acts, hipStream_t s);
 hipError_t launch_gemv_q8_grouped(const DevWeight &w, const DevWeight *wtab, float *out, const DevWeight *wtab2, float *out2,
                                   const void *acts, int n_tile_max, const MoeTile *tiles, const int *n_tiles, hipStream_t s);
+// Grouped GEMM: for every tile (expert e, slots r0 ..): out[r0 + m, :] =
+// epi(A[gather ? gather[r0 + m] : r0 + m, :] . wtab[e]^T).  `w` gives the
+// dtype and shape shared by all experts; wtab is a device array of
+// DevWeight; a_rows: rows of A (bounds the loads); max_tiles bounds
+// n_tiles_dev[0].
 hipError_t launch_gemm_f16_grouped(const DevWeight &w, const DevWeight *wtab, const void *a_f16, size_t a_rows,
                                    const int *gather, const MoeTile *tiles, const int *n_tiles_dev, int max_tiles,
                                    int bm, int epi, void *out, const float *aux, hipStream_t s);
