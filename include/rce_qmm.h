@@ -226,7 +226,9 @@ rce_qmm_status rce_qmm_mm_batched_dev(rce_qmm_context *ctx, const void *a_dev, u
  * fixed device array of RCE_QMM_NOALLOC_SCRATCH_BYTES that each GPU the
  * library runs on holds until the process ends; a call that needs more
  * returns RCE_QMM_BAD_SHAPE.  All calls on one GPU share that array:
- * calls that overlap on one GPU (other streams, other contexts) race. */
+ * calls that overlap on one GPU (other streams, other contexts) race.
+ * F16_MFMA calls of few tokens also use a buffer allocated with the context
+ * (the sums of their K slices). */
 #define RCE_QMM_NOALLOC_SCRATCH_BYTES (16u << 20)
 rce_qmm_status rce_qmm_mm_batched_dev_noalloc(rce_qmm_context *ctx, const void *a_dev, uint32_t a_dtype,
                                               size_t t_rows, const rce_qmm_weight *w, float *out_dev,

@@ -67,7 +67,10 @@ struct rce_qmm_context {
     std::atomic<int> refs{1};
     rce_qmm_abi::Scratch a_in, a_f32, out;
     rce_qmm_abi::Scratch a_f16;  // f32 activations rounded to f16 for the MFMA GEMM
-    rce_qmm_abi::Scratch parts;  // sums of the GEMM's K slices (at most a 64 x 64 tile's per CU: 4 MiB)
+    // Sums of the GEMM's K slices: gemm_f16_parts_bytes(), the most any call
+    // needs, allocated with the context and never moved, so a call recorded
+    // into a graph stays valid whatever calls follow it.
+    rce_qmm_abi::Scratch parts;
     rce_qmm_abi::Scratch act_q;  // several tokens' Q8 activations, quantized once per launch
     // grouped experts: grouping metadata, expert tables, stage buffers
     rce_qmm_abi::Scratch moe_meta, moe_wtab, moe_x, moe_h, moe_h16, moe_y, moe_u;

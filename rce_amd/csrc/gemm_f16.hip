@@ -324,7 +324,7 @@ struct Q6K {
 template <class T, class Fmt, int EPI>
 __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__restrict__ A, uint32_t a_bytes,
                                           void *__restrict__ out_v, const float *__restrict__ aux, size_t m0,
-                                          int rows, size_t n0, const int *arow, unsigned char *lds, int gb = 0, int slice_groups = 0, bool add = false) {
+                                          int rows, size_t n0, const int *arow, unsigned char *lds, int gb = 0, int slice_groups = 0) {
     constexpr int BM = T::BM, BN = T::BN, RB = T::RB, CB = T::CB, NS = T::NS, NH = Fmt::NH;
     constexpr int A_STAGE = T::A_STAGE, W_HALF = T::W_HALF, W_GROUP = T::W_GROUP;
     constexpr int OFF_W = T::OFF_W;
@@ -703,11 +703,8 @@ __device__ __forceinline__ void gemm_tile(const DevWeight &w, const _Float16 *__
                     const int m = 32 * orb + 8 * rq + 4 * h + e;
                     if (m < rows && col < N) {
                         const size_t o = (m0 + m) * N + col;
-                        if constexpr (EPI == GEPI_F32) {
+                        if constexpr (EPI == GEPI_F32 || EPI == GEPI_SLICE) {
                             static_cast<float *>(out_v)[o] = sum[e];
-                        } else if constexpr (EPI == GEPI_SLICE) {
-                            float *op = static_cast<float *>(out_v) + o;
-                            *op = add ? *op + sum[e] : sum[e];
                         } else if constexpr (EPI == GEPI_SILU_F16) {  // rce-qwen36-moe/src/lib.rs L459-461
                             static_cast<_Float16 *>(out_v)[o] = (_Float16)silu_mfma(sum[e]);
                         } else {  // silu(g) * u, rce-qwen36-moe/src/lib.rs L667-676
@@ -729,7 +726,7 @@ __global__ __launch_bounds__(NT) void k_gemm_f16(DevWeight w_arg, const _Float16
                                                  const int *__restrict__ gather, size_t M, uint32_t a_bytes,
                                                  void *__restrict__ out_v, const float *__restrict__ aux, int m_tiles,
                                                  const MoeTile *__restrict__ tiles, const int *__restrict__ n_tiles,
-                                                 const DevWeight *__restrict__ wtab, int slice0, int slices) {
+                                                 const DevWeight *__restrict__ wtab, int slices) {
     using T = Tile<BM_, Fmt, BN_>;
     constexpr int BM = T::BM;
     extern __shared__ __align__(16) unsigned char lds[];
@@ -769,14 +766,12 @@ __global__ __launch_bounds__(NT) void k_gemm_f16(DevWeight w_arg, const _Float16
     }
     __syncthreads();
     const size_t n0 = (size_t)nt * T::BN;
-    // GEPI_SLICE: this block's K slice is slice0 + blockIdx.y of `slices`.  A
-    // launch of several writes slice y's sums to rows y M .. of out_v; one of
-    // a single later slice adds to out_v.
+    // GEPI_SLICE: this block's K slice is blockIdx.y of `slices`; slice y's
+    // sums go to rows y M .. of out_v.
     if constexpr (EPI == GEPI_SLICE) {
-        const int groups = (int)(w.n_cols / (4 * KC)), slice = slice0 + (int)blockIdx.y;
+        const int groups = (int)(w.n_cols / (4 * KC)), slice = (int)blockIdx.y;
         const int gb = groups * slice / slices, ng = groups * (slice + 1) / slices - gb;
-        gemm_tile<T, Fmt, EPI>(w, A, a_bytes, out_v, aux, m0 + blockIdx.y * M, rows, n0, arow, lds, gb, ng,
-                               gridDim.y == 1 && slice > 0);
+        gemm_tile<T, Fmt, EPI>(w, A, a_bytes, out_v, aux, m0 + blockIdx.y * M, rows, n0, arow, lds, gb, ng);
         return;
     }
     // A 96- or 128-row tile that holds at most 64 rows (a grouped tile whose
@@ -837,17 +832,16 @@ hipError_t set_lds_attr() {
     return ensure_lds_limit((const void *)k_gemm_f16<Fmt, BM, EPI, BN_>, Tile<BM, Fmt, BN_>::LDS);
 }
 
-// K slices slice0 .. slice0 + count - 1 of `slices` (EPI GEPI_SLICE), or all of K.
+// All of K, or each of its slices (EPI GEPI_SLICE).
 template <class Fmt, int BM, int BN_ = 0, int EPI = GEPI_F32>
-hipError_t launch_fmt(const DevWeight &w, const _Float16 *a, size_t M, float *out, hipStream_t s, int slice0 = 0,
-                      int count = 1, int slices = 1) {
+hipError_t launch_fmt(const DevWeight &w, const _Float16 *a, size_t M, float *out, hipStream_t s, int slices = 1) {
     using T = Tile<BM, Fmt, BN_>;
     const int m_tiles = (int)((M + T::BM - 1) / T::BM), n_tiles = (int)((w.n_rows + T::BN - 1) / T::BN);
     hipError_t e = set_lds_attr<Fmt, BM, EPI, BN_>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_gemm_f16<Fmt, BM, EPI, BN_>), dim3(m_tiles * n_tiles, count), dim3(NT), T::LDS, s, w, a,
+    hipLaunchKernelGGL((k_gemm_f16<Fmt, BM, EPI, BN_>), dim3(m_tiles * n_tiles, slices), dim3(NT), T::LDS, s, w, a,
                        (const int *)nullptr, M, (uint32_t)(M * w.n_cols * 2), (void *)out, (const float *)nullptr,
-                       m_tiles, (const MoeTile *)nullptr, (const int *)nullptr, (const DevWeight *)nullptr, slice0, slices);
+                       m_tiles, (const MoeTile *)nullptr, (const int *)nullptr, (const DevWeight *)nullptr, slices);
     return hipGetLastError();
 }
 
@@ -860,8 +854,7 @@ hipError_t launch_fmt_grouped(const DevWeight &w, const DevWeight *wtab, const _
     hipError_t e = set_lds_attr<Fmt, BM, EPI>();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_gemm_f16<Fmt, BM, EPI>), dim3(grouped_grid(max_tiles, n_tiles)), dim3(NT), T::LDS, s, w, a,
-                       gather, a_rows, (uint32_t)(a_rows * w.n_cols * 2), out, aux, max_tiles, tiles, n_tiles_dev, wtab, 0,
-                       1);
+                       gather, a_rows, (uint32_t)(a_rows * w.n_cols * 2), out, aux, max_tiles, tiles, n_tiles_dev, wtab, 1);
     return hipGetLastError();
 }
 
@@ -1073,44 +1066,36 @@ int gemm_slices(const DevWeight &w, size_t M, const GemmTile &t, size_t cus) {
 
 }  // namespace
 
-size_t gemm_f16_slice_bytes(const DevWeight &w, size_t M) {
-    if (M == 0 || w.n_rows == 0 || !gemm_shape_ok(M, w) || !(gemm_supports(w.dtype, w.n_cols) || gemm_q8_supports(w.dtype, w.n_cols)))
-        return 0;
-    const size_t cus = cu_count() ? (size_t)cu_count() : 256;
-    const int sl = gemm_slices(w, M, pick_gemm_tile(w, M, cus, 0), cus);
-    return sl == 1 ? 0 : (size_t)sl * M * w.n_rows * sizeof(float);
-}
+// Slices times 64 x 64 tiles are at most the CUs (gemm_slices).
+size_t gemm_f16_parts_bytes() { return (cu_count() ? (size_t)cu_count() : 256) * 64 * 64 * sizeof(float); }
 
-hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, int bm, float *parts) {
+hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, float *parts, int bm) {
     if (M == 0 || w.n_rows == 0) return hipSuccess;
     if (!gemm_shape_ok(M, w)) return hipErrorInvalidValue;
     const _Float16 *a = static_cast<const _Float16 *>(a_f16);
     const size_t cus = cu_count() ? (size_t)cu_count() : 256;
     const GemmTile g = pick_gemm_tile(w, M, cus, bm);
     const int sl = bm == 0 ? gemm_slices(w, M, g, cus) : 1;
-    // without room for the slices' sums: slice after slice, each adding to
-    // the output (the same bits)
-    float *o = sl > 1 && parts ? parts : out;
-    const int count = sl > 1 && parts ? sl : 1;
+    if (sl > 1 && !parts) return hipErrorInvalidValue;
     hipError_t e = hipSuccess;
     auto launch = [&](auto fmt, auto q8_layout) {
         using F = decltype(fmt);
         if (sl > 1) {  // 64 x 64 tiles
-            for (int y = 0; y < sl && e == hipSuccess; y += count) e = launch_fmt<F, 64, 64, GEPI_SLICE>(w, a, M, o, s, y, count, sl);
+            e = launch_fmt<F, 64, 64, GEPI_SLICE>(w, a, M, parts, s, sl);
         } else if (g.sq64) {
-            e = launch_fmt<F, 64, 64>(w, a, M, o, s);
+            e = launch_fmt<F, 64, 64>(w, a, M, out, s);
         } else if (g.bm == 128) {
-            e = launch_fmt<F, 128>(w, a, M, o, s);
+            e = launch_fmt<F, 128>(w, a, M, out, s);
         } else if constexpr (decltype(q8_layout)::value) {
             e = hipErrorInvalidValue;
         } else {
-            e = g.bm == 64 ? launch_fmt<F, 64>(w, a, M, o, s) : (g.bm == 96 ? launch_fmt<F, 96>(w, a, M, o, s) : hipErrorInvalidValue);
+            e = g.bm == 64 ? launch_fmt<F, 64>(w, a, M, out, s) : (g.bm == 96 ? launch_fmt<F, 96>(w, a, M, out, s) : hipErrorInvalidValue);
         }
     };
     if (w.dtype == T_Q8_0) launch(Q80{}, ic<1>{});
     else if (w.dtype == T_Q6_K) launch(Q6K{}, ic<1>{});
     else if (!with_fmt(w.dtype, [&](auto fmt) { launch(fmt, ic<0>{}); })) e = hipErrorInvalidValue;
-    if (e != hipSuccess || count == 1) return e;
+    if (e != hipSuccess || sl == 1) return e;
     const size_t n = M * w.n_rows;
     if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(parts)) % 16 == 0)
         hipLaunchKernelGGL(k_sum_slices<f32x4>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,

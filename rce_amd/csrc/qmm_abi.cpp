@@ -68,7 +68,6 @@ struct BatchedScratch {
     float *a_f32 = nullptr;       // F16 activations widened to f32 (EXACT, Q8)
     unsigned char *act_q = nullptr;  // Q8 activations of several tokens, quantized once
     void *a_f16 = nullptr;        // F32 activations rounded to f16 (F16_MFMA)
-    float *parts = nullptr;       // the sums of the GEMM's K slices (F16_MFMA, short M)
 };
 
 }  // namespace
@@ -90,7 +89,7 @@ namespace {
 
 // The prefill GEMM; f32 activations are rounded to f16 first (into sc.a_f16).
 rce_qmm_status run_gemm(const void *a_dev, bool a_f16, size_t t_rows, const DevWeight &dw, float *out_dev,
-                        const BatchedScratch &sc, hipStream_t s) {
+                        const BatchedScratch &sc, float *parts, hipStream_t s) {
     const void *a = a_dev;
     if (!a_f16) {
         HIP_TRY(launch_f32_to_f16(static_cast<const float *>(a_dev), sc.a_f16, t_rows * dw.n_cols, s));
@@ -112,7 +111,7 @@ rce_qmm_status run_gemm(const void *a_dev, bool a_f16, size_t t_rows, const DevW
         const _Float16 *a16 = static_cast<const _Float16 *>(a);
         for (size_t r0 = 0; r0 < t_rows; r0 += max_rows) {
             const size_t rows = t_rows - r0 < max_rows ? t_rows - r0 : max_rows;
-            HIP_TRY(launch_gemm_f16(dw, a16 + r0 * k, rows, out_dev + r0 * dw.n_rows, s, 0, rows == t_rows ? sc.parts : nullptr));
+            HIP_TRY(launch_gemm_f16(dw, a16 + r0 * k, rows, out_dev + r0 * dw.n_rows, s, parts));
         }
     } else {
         HIP_TRY(launch_gemm_gen(dw, a, t_rows, out_dev, s));
@@ -153,19 +152,6 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
         else q8_b = b;
     }
     const size_t f16_b = mfma && a_dtype == T_F32 ? t_rows * k * 2 : 0;
-    // The GEMM's K slices: without room for their sums (the fixed scratch; a
-    // buffer to grow under stream capture) they run one after another.
-    size_t part_b = mfma && !gemm_wide_preferred(dw, t_rows) ? gemm_f16_slice_bytes(dw, t_rows) : 0;
-    if (part_b && fixed && align_up(f16_b, 256) + align_up(part_b, 256) > fixed_cap) part_b = 0;
-    if (part_b && !fixed && ctx->parts.cap < part_b) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-            (void)hipGetLastError();
-            part_b = 0;
-        } else if (cap != hipStreamCaptureStatusNone) {
-            part_b = 0;
-        }
-    }
     BatchedScratch sc;
     rce_qmm_status st;
     if (fixed) {
@@ -177,7 +163,6 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
         if (f32_b) { sc.a_f32 = reinterpret_cast<float *>(p); p += align_up(f32_b, 256); }
         if (q8_b) { sc.act_q = p; p += align_up(q8_b, 256); }
         if (f16_b) { sc.a_f16 = p; p += align_up(f16_b, 256); }
-        if (part_b) { sc.parts = reinterpret_cast<float *>(p); p += align_up(part_b, 256); }
     } else {
         if (f32_b) {
             if ((st = ensure(ctx, ctx->a_f32, f32_b, s))) return st;
@@ -191,12 +176,8 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
             if ((st = ensure(ctx, ctx->a_f16, f16_b, s))) return st;
             sc.a_f16 = ctx->a_f16.p;
         }
-        if (part_b) {
-            if ((st = ensure(ctx, ctx->parts, part_b, s))) return st;
-            sc.parts = static_cast<float *>(ctx->parts.p);
-        }
     }
-    if (mfma) return run_gemm(a_dev, a_dtype == T_F16, t_rows, dw, out_dev, sc, s);
+    if (mfma) return run_gemm(a_dev, a_dtype == T_F16, t_rows, dw, out_dev, sc, static_cast<float *>(ctx->parts.p), s);
     const float *a32 = static_cast<const float *>(a_dev);
     if (widen) {
         HIP_TRY(launch_f16_to_f32(static_cast<const uint16_t *>(a_dev), sc.a_f32, t_rows * k, s));
@@ -336,6 +317,10 @@ rce_qmm_status rce_qmm_context_create(int device, rce_qmm_context **out) {
     }
     c->device = device;
     c->stream = s;
+    if ((st = ensure(c, c->parts, rce_qmm::gemm_f16_parts_bytes(), nullptr))) {
+        context_release(c);
+        return st;
+    }
     *out = c;
     return RCE_QMM_OK;
 }

@@ -380,12 +380,10 @@ bool gemm_q8_supports(uint32_t dtype, size_t n_cols);
 bool gemm_shape_ok(size_t a_rows, const DevWeight &w);
 // bm: output tile rows, 64 (tile 64 x 128), 96 (96 x 128) or 128 (128 x 64);
 // 0 = by M.
-// parts: gemm_f16_slice_bytes(w, M) bytes for the sums of K slices (null: the
-// slices run one after another, with the same bits).
-hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, int bm = 0,
-                           float *parts = nullptr);
-// The bytes launch_gemm_f16 would use for K slices (0: it uses none).
-size_t gemm_f16_slice_bytes(const DevWeight &w, size_t M);
+// parts: gemm_f16_parts_bytes() bytes for the sums of K slices.
+hipError_t launch_gemm_f16(const DevWeight &w, const void *a_f16, size_t M, float *out, hipStream_t s, float *parts, int bm = 0);
+// The most bytes the K slices of any launch on the current device need.
+size_t gemm_f16_parts_bytes();
 // The other formats' prefill GEMM (gemm_gen.hip): Q8_0, Q5_0, Q4_1, F16 (K
 // a multiple of 64), Q5_K, Q6_K (K a multiple of 256); nibble_forms also
 // admits Q4_0 and Q4_K (the same generic form, for cross-checks).  A must

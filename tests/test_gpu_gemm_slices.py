@@ -1,7 +1,7 @@
 """GPU checks of the prefill GEMM's K slices (gemm_f16.hip, short M): against
-float64 products of the dequantized weights, run to run, and where the slices'
-sums do not fit the fixed scratch (slice after slice into the output) bit for
-bit the same as where they do."""
+float64 products of the dequantized weights, run to run, and through the
+no-allocation entry point next to a scratch that the activations nearly
+fill."""
 import numpy as np
 import pytest
 
@@ -36,7 +36,7 @@ def test_slices(ctx, dt, m, n, k):
     w.close()
 
 
-def test_without_room_for_the_sums(ctx):
+def test_beside_a_full_scratch(ctx):
     m, n, k = 256, 1100, 24576  # 12.6 MB of binary16 activations and 4.5 MB of sums against 16 MiB
     rng = np.random.default_rng(3)
     w = rce_amd.QuantWeight.from_owned_bytes(ctx, weight_bytes(rng, O.Q4_0, n, k), O.Q4_0, n, k)
