@@ -87,6 +87,14 @@ size_t rce_qmm_abi::batched_scratch_bytes(const DevWeight &dw, uint32_t a_dtype,
 
 namespace {
 
+// Whether `s` is being recorded into a graph.
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // The prefill GEMM; f32 activations are rounded to f16 first (into sc.a_f16).
 rce_qmm_status run_gemm(const void *a_dev, bool a_f16, size_t t_rows, const DevWeight &dw, float *out_dev,
                         const BatchedScratch &sc, float *parts, hipStream_t s) {
@@ -146,9 +154,12 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     // Q8 on the int8 matrix cores: whole tiles of 16 tokens; where those do
     // not fit the fixed scratch, the form that needs the documented bytes
     bool mma = mode == RCE_QMM_MODE_Q8 && gemv_q8_mfma_supports(dw.dtype, k, t_rows) && gemv_q8_mfma_preferred(dw, t_rows);
+    // Being recorded, neither where those would have to grow the context's
+    // buffer nor where the other form needs none: a call recorded without
+    // scratch stays valid whatever calls follow it.
     if (mma) {
         const size_t b = (t_rows + 15) / 16 * gemv_q8_tile_bytes(k);
-        if (fixed && align_up(f32_b, 256) + align_up(b, 256) > fixed_cap) mma = false;
+        if (fixed ? align_up(f32_b, 256) + align_up(b, 256) > fixed_cap : (!preq || ctx->act_q.cap < b) && capturing(s)) mma = false;
         else q8_b = b;
     }
     const size_t f16_b = mfma && a_dtype == T_F32 ? t_rows * k * 2 : 0;

@@ -63,3 +63,27 @@ def test_k_slices(record):
 
         replay_equals_eager(c, record, between, xa, G.F16, 16, w, Mode.F16_MFMA)
         xa.free(); big.free(); w.close()
+
+
+@pytest.mark.parametrize("record", ["cold", "warm"])
+@pytest.mark.parametrize("dt", [O.Q5_0, O.Q4_1])
+def test_q8_formats_without_scratch(monkeypatch, dt, record):
+    """32 tokens recorded for formats whose decode kernels quantize inside
+    their blocks, 200 (a larger workspace of the matrix-core form) and new
+    allocations between the replays."""
+    print(f"capture q8 dtype={dt} {record}", flush=True)
+    monkeypatch.setenv("RCE_QMM_Q8_MFMA", "2")
+    rng = np.random.default_rng(2)
+    with rce_amd.Context(0) as c:
+        w = weight(c, rng, dt, 512, 2048)
+        xa = rce_amd.DeviceBuffer.from_numpy(c, rng.standard_normal((200, 2048)).astype(F32))
+        big = rce_amd.DeviceBuffer(c, 200 * 512 * 4)
+
+        def between():
+            rce_amd.mm_batched_dev(c, xa.ptr, G.F32, 200, w, big.ptr, Mode.Q8)
+            c.synchronize()
+            for nbytes in (81920, 1 << 17):
+                rce_amd.DeviceBuffer.from_numpy(c, np.full(nbytes, 255, np.uint8)).free()
+
+        replay_equals_eager(c, record, between, xa, G.F32, 32, w, Mode.Q8)
+        xa.free(); big.free(); w.close()
