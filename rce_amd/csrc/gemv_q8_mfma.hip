@@ -40,6 +40,8 @@
 #include "mfma_util.h"
 #include "qmm_gemv_kernels.h"
 
+#include <algorithm>
+
 namespace rce_qmm {
 namespace {
 
@@ -519,11 +521,26 @@ __global__ __launch_bounds__(512) void k_quantize_tiles(const float *__restrict_
             make_uint2(__float_as_uint((float)(_Float16)d), ((uint32_t)half & 0xFFFFu) | ((uint32_t)other << 16));
 }
 
+// HIP takes fewer than 2^32 threads in a dimension of a grid.
+constexpr size_t MAX_BLOCKS = ((size_t)1 << 24) - 1;
+// Slices of 16 rows, padded to whole turns of the XCDs.
+size_t row_slices(const DevWeight &w) { return ((w.n_rows + 15) / 16 + 7) / 8 * 8; }
+
+bool weight_ok(const DevWeight &w) {
+    switch (w.dtype) {
+    case T_Q4_0: case T_Q8_0: case T_Q5_0: case T_Q4_1: case T_Q4_K: case T_Q5_K: case T_Q6_K: break;
+    default: return false;
+    }
+    // a wave's 16 rows (a 64-row group) within 32-bit offsets
+    return gpu_supports(w.dtype, w.n_cols, 1) && w.n_cols % QK == 0 && 16 * w.row_stride < ((size_t)1 << 31) &&
+           w.group_stride < ((size_t)1 << 31);
+}
+
 template <Q8Fmt F>
 hipError_t launch_fmt(const Q8Out &o0, const Q8Out &o1, int nw, const unsigned char *acts, int T, int n_tile_max,
                       const MoeTile *tiles, const int *n_tiles, hipStream_t s) {
-    const size_t slices = (o0.w.n_rows + 15) / 16, blocks = (slices + 7) / 8 * 8 * (size_t)n_tile_max;
-    if (blocks >= (size_t)1 << 31) return hipErrorInvalidValue;
+    const size_t blocks = row_slices(o0.w) * (size_t)n_tile_max;
+    if (blocks > MAX_BLOCKS) return hipErrorInvalidValue;
     constexpr int LDS = QFmt<F>::LDS;
     hipError_t e = ensure_lds_limit((const void *)k_gemv_q8_mfma<F>, LDS);
     if (e != hipSuccess) return e;
@@ -534,8 +551,7 @@ hipError_t launch_fmt(const Q8Out &o0, const Q8Out &o1, int nw, const unsigned c
 
 hipError_t launch_any(const Q8Out &o0, const Q8Out &o1, int nw, const unsigned char *acts, int T, int n_tile_max,
                       const MoeTile *tiles, const int *n_tiles, hipStream_t s) {
-    // a wave's 16 rows (a 64-row group) within 32-bit offsets
-    if (16 * o0.w.row_stride >= ((size_t)1 << 31) || o0.w.group_stride >= ((size_t)1 << 31)) return hipErrorInvalidValue;
+    if (!weight_ok(o0.w)) return hipErrorInvalidValue;
     switch (o0.w.dtype) {
     case T_Q4_0: return launch_fmt<QF_Q4_0>(o0, o1, nw, acts, T, n_tile_max, tiles, n_tiles, s);
     case T_Q8_0: return launch_fmt<QF_Q8_0>(o0, o1, nw, acts, T, n_tile_max, tiles, n_tiles, s);
@@ -550,13 +566,13 @@ hipError_t launch_any(const Q8Out &o0, const Q8Out &o1, int nw, const unsigned c
 
 }  // namespace
 
-// The formats and widths of this form (t_rows: the decode kernels' own bound).
-bool gemv_q8_mfma_supports(uint32_t dtype, size_t n_cols, size_t t_rows) {
-    switch (dtype) {
-    case T_Q4_0: case T_Q8_0: case T_Q5_0: case T_Q4_1: case T_Q4_K: case T_Q5_K: case T_Q6_K: break;
-    default: return false;
-    }
-    return gpu_supports(dtype, n_cols, 1) && n_cols % QK == 0 && t_rows >= 2 && t_rows <= 65535 * 8;
+// The formats and shapes of this form (t_rows: the decode kernels' own bound).
+bool gemv_q8_mfma_supports(const DevWeight &w, size_t t_rows) {
+    return weight_ok(w) && row_slices(w) <= MAX_BLOCKS && t_rows >= 2 && t_rows <= 65535 * 8;
+}
+
+bool gemv_q8_grouped_supports(const DevWeight &w, size_t n_tile_max) {
+    return weight_ok(w) && n_tile_max <= 65535 && row_slices(w) * n_tile_max <= MAX_BLOCKS;
 }
 
 // Where this form is the faster one, by estimates fitted to both forms'
@@ -610,12 +626,20 @@ hipError_t launch_quantize_tiles(int src, const float *a, const float *a2, size_
 
 hipError_t launch_gemv_q8_mfma(const DevWeight &w, const float *a, size_t t_rows, float *out, void *acts, hipStream_t s) {
     if (t_rows == 0 || w.n_rows == 0) return hipSuccess;
-    if (!gemv_q8_mfma_supports(w.dtype, w.n_cols, t_rows)) return hipErrorInvalidValue;
+    if (!gemv_q8_mfma_supports(w, t_rows)) return hipErrorInvalidValue;
     const int nt = (int)((t_rows + 15) / 16);
     hipError_t e = launch_quantize_tiles(Q8SRC_ROWS, a, nullptr, w.n_cols, t_rows, nt, nullptr, nullptr, nullptr, acts, s);
     if (e != hipSuccess) return e;
-    const Q8Out o{w, nullptr, out};
-    return launch_any(o, o, 1, static_cast<const unsigned char *>(acts), (int)t_rows, nt, nullptr, nullptr, s);
+    // as many tiles a launch as its grid takes
+    const int per = (int)std::min<size_t>(MAX_BLOCKS / row_slices(w), (size_t)nt);
+    const unsigned char *q = static_cast<const unsigned char *>(acts);
+    for (int g = 0; g < nt && e == hipSuccess; g += per) {
+        const size_t t0 = 16 * (size_t)g;
+        const Q8Out o{w, nullptr, out + t0 * w.n_rows};
+        e = launch_any(o, o, 1, q + (size_t)g * gemv_q8_tile_bytes(w.n_cols), (int)(t_rows - t0), std::min(per, nt - g), nullptr,
+                       nullptr, s);
+    }
+    return e;
 }
 
 hipError_t launch_gemv_q8_grouped(const DevWeight &w, const DevWeight *wtab, float *out, const DevWeight *wtab2, float *out2,

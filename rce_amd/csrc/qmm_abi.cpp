@@ -153,7 +153,7 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     size_t q8_b = preq ? t_rows * (k + k / 8 + k / 4) : 0;  // xq, dx, s16
     // Q8 on the int8 matrix cores: whole tiles of 16 tokens; where those do
     // not fit the fixed scratch, the form that needs the documented bytes
-    bool mma = mode == RCE_QMM_MODE_Q8 && gemv_q8_mfma_supports(dw.dtype, k, t_rows) && gemv_q8_mfma_preferred(dw, t_rows);
+    bool mma = mode == RCE_QMM_MODE_Q8 && gemv_q8_mfma_supports(dw, t_rows) && gemv_q8_mfma_preferred(dw, t_rows);
     // Being recorded, neither where those would have to grow the context's
     // buffer nor where the other form needs none: a call recorded without
     // scratch stays valid whatever calls follow it.
@@ -633,8 +633,9 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
         const bool args = n_expert <= MOE_ARG_EXPERTS && n_pairs + n_expert <= 65535;
         if (args && gemv_grouped_supports(a1.dtype, d_model, (int)mode) && gemv_grouped_supports(a2.dtype, d_ff, (int)mode))
             form = BY_TILE;
-        if (args && mode == RCE_QMM_MODE_Q8 && gemv_q8_mfma_supports(a1.dtype, d_model, 2) &&
-            gemv_q8_mfma_supports(a2.dtype, d_ff, 2) && moe_q8_mfma_preferred(per_expert, a1.dtype == T_Q6_K || a2.dtype == T_Q6_K, form != BY_EXPERT))
+        const size_t tiles16 = n_pairs / 16 + n_expert;
+        if (args && mode == RCE_QMM_MODE_Q8 && gemv_q8_grouped_supports(a1, tiles16) && gemv_q8_grouped_supports(a2, tiles16) &&
+            moe_q8_mfma_preferred(per_expert, a1.dtype == T_Q6_K || a2.dtype == T_Q6_K, form != BY_EXPERT))
             form = Q8_MFMA;
     }
     // tile rows: for the average rows per expert in the grouped GEMM (the

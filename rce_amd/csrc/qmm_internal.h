@@ -332,7 +332,7 @@ bool gemv_q8_pre_supports(uint32_t dtype, size_t n_cols, size_t t_rows);
 // each.  Chosen where it is faster (gemv_q8_mfma_preferred);
 // RCE_QMM_Q8_MFMA=0 turns it off, =2 forces it wherever it applies (same
 // bits either way).
-bool gemv_q8_mfma_supports(uint32_t dtype, size_t n_cols, size_t t_rows);
+bool gemv_q8_mfma_supports(const DevWeight &w, size_t t_rows);
 bool gemv_q8_mfma_preferred(const DevWeight &w, size_t t_rows);
 size_t gemv_q8_tile_bytes(size_t n_cols);
 hipError_t launch_gemv_q8_mfma(const DevWeight &w, const float *a, size_t t_rows, float *out, void *acts, hipStream_t s);
@@ -511,7 +511,9 @@ enum GemmEpilogue { GEPI_F32 = 0, GEPI_SILU_F16 = 1, GEPI_SWIGLU_F16 = 2, GEPI_S
 // slots' tokens (tok_of_slot) or plain rows, Q8SRC_SILU silu(a[slot]),
 // Q8SRC_SWIGLU silu(a[slot]) * a2[slot]; launch_gemv_q8_grouped forms out[slot] =
 // wtab[expert] . acts (and out2 with wtab2, a second matrix of the same
-// shape).  At most 65535 tiles.
+// shape).  gemv_q8_grouped_supports: whether w and the most tiles a call can
+// have are within the launches' limits.
+bool gemv_q8_grouped_supports(const DevWeight &w, size_t n_tile_max);
 enum : int { Q8SRC_ROWS = 0, Q8SRC_SILU = 1, Q8SRC_SWIGLU = 2 };
 hipError_t launch_quantize_tiles(int src, const float *a, const float *a2, size_t k, size_t t_rows, int n_tile_max,
                                  const MoeTile *tiles, const int *n_tiles, const int *tok_of_slot, void *acts, hipStream_t s);

@@ -1,6 +1,8 @@
 """GPU parity of the int8 matrix-core form of the Q8 mode (gemv_q8_mfma.hip),
 forced on every case: the same bits as the oracle's Q8 restatement, at the
 edges of its tiles (16 tokens, 64 rows, stages of 256 with a ring of three)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -8,6 +10,7 @@ import oracle as O
 import rce_amd
 from rand_blocks import rand_blocks
 from rce_amd import Mode
+from rce_amd._lib import check, lib
 from test_gpu_gemv import bits, run_dev
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +38,25 @@ def test_bit_identical(ctx, monkeypatch, dt, n, k, t):
     want = O.mm_batched_q8(x, b, dt, n, k)
     assert np.array_equal(bits(got), bits(want)), f"{np.sum(bits(got) != bits(want))} values differ"
     w.close()
+
+
+def test_outputs_past_the_grid_limit(ctx, monkeypatch):
+    """2^32 and more outputs: 65536 rows times 65552 tokens are 2^24 + 4096
+    blocks of 256 threads, more threads than a grid dimension takes.  The first and last
+    tokens have the bits of a call of their own."""
+    monkeypatch.setenv("RCE_QMM_Q8_MFMA", "2")
+    n, k, t = 65536, 256, 65552
+    print(f"q8 mfma n={n} k={k} t={t}", flush=True)
+    rng = np.random.default_rng(9)
+    b = rand_blocks(rng, O.Q8_0, n, k)
+    w = rce_amd.QuantWeight.from_owned_bytes(ctx, b, O.Q8_0, n, k)
+    x = rng.standard_normal((t, k)).astype(np.float32)
+    xa = rce_amd.DeviceBuffer.from_numpy(ctx, x)
+    out = rce_amd.DeviceBuffer(ctx, 4 * n * t)
+    rce_amd.mm_batched_dev(ctx, xa.ptr, rce_amd.GgufDtype.F32, t, w, out.ptr, Mode.Q8)
+    ctx.synchronize()
+    for t0 in (0, t - 32, t - 4):  # the first tokens, both sides of the second launch's first tile
+        got = np.empty((4, n), np.float32)
+        check(lib().rce_qmm_memcpy_d2h(ctx.handle, ctypes.c_void_p(got.ctypes.data), ctypes.c_void_p(out.ptr + 4 * n * t0), got.nbytes))
+        assert np.array_equal(bits(got), bits(run_dev(ctx, w, x[t0:t0 + 4], Mode.Q8))), t0
+    xa.free(); out.free(); w.close()
