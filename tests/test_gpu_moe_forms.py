@@ -76,3 +76,19 @@ def test_bad_id_is_an_error_and_the_next_call_is_clean(ctx, mode):
         run_moe(ctx, w1, w2, O.Q4_0, 256, 512, x, bad, gw, mode)
     got = run_moe(ctx, w1, w2, O.Q4_0, 256, 512, x, ids, gw, mode)
     assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q4_0, 512, ids, gw, q8=mode == Mode.Q8, silu_dev=True))
+
+
+@pytest.mark.parametrize("mma", ["0", "2"])
+def test_many_experts_expert_by_expert_q8(ctx, monkeypatch, mma):
+    """One expert past the kernel arguments' table, forty tokens on one of
+    them: its products on the matrix cores and on the decode kernels."""
+    monkeypatch.setenv("RCE_QMM_Q8_MFMA", mma)
+    print(f"moe expert by expert mma={mma}", flush=True)
+    rng = np.random.default_rng(6)
+    E, dm, dff, t = 65, 256, 512, 40
+    w1, w2 = experts(rng, O.Q4_0, E, dff, dm), experts(rng, O.Q4_0, E, dm, dff)
+    x = rng.standard_normal((t, dm)).astype(np.float32)
+    ids = np.stack([np.full(t, 64), np.arange(t) % 64], 1).astype(np.int32)
+    gw = np.full((t, 2), 0.5, np.float32)
+    got = run_moe(ctx, w1, w2, O.Q4_0, dm, dff, x, ids, gw, Mode.Q8)
+    assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q4_0, dff, ids, gw, q8=True, silu_dev=True))
