@@ -576,35 +576,56 @@ bool gemv_q8_grouped_supports(const DevWeight &w, size_t n_tile_max) {
 }
 
 // Where this form is the faster one, by estimates fitted to both forms'
-// times (us, quantization included) at 2-64 tokens, N 1024-14336, K
-// 2048-8192.  With M = N K / 10^6 and tiles of 16 tokens:
-//   decode kernels: 7.3 + 0.021 M per token; Q6_K 5 + 0.05 M (two tokens per
-//     block, and its super-block's scales per token); a row of more than 256
-//     units (blocks of 32: K > 8192, 64-groups: K > 16384) 4 + 0.2 M from 4
-//     tokens on (no pre-quantized form there);
-//   this form: the larger of its chain over K, 5 + 1.2 (K-quants), 1.6
-//     (blocks of 32), 2.7 (Q6_K) per 1024 of K, and its arithmetic, 5 + 0.18 M
-//     (Q6_K 0.43) per tile.
-// Measured there, decode kernels / this form: Q4_K 14336x4096 at 8 / 16 / 32 /
-// 64 tokens 19.2 / 28.2 / 47.4 / 87.9 against 17.9 / 18.3 / 25.9 / 44.2; Q4_0
-// 11008x4096 at 8 / 16 / 32 14.0 / 20.7 / 33.4 against 15.6 / 15.8 / 24.2; Q4_0
-// 4096x14336 at 4 / 16 / 64 50 / 183 / 739 against 28 / 28 / 48; Q6_K 2048x5632
-// at 8 / 24 / 32 11.5 / 18.5 / 22.0 against 20.2 / 20.6 / 20.6, 11008x4096 at 8 /
-// 12 / 32 24.6 / 33.0 / 76 against 25.2 / 25.4 / 41; Q8_0 512x8192 at 32
-// 10.3 against 17.7.
+// times (us, quantization included) at 2-128 tokens, N 512-14336, K
+// 512-14336, every format.  With t tokens, M = N K / 10^6 and tiles of 16 tokens:
+//   decode kernels, the formats quantized once per launch (a row of at most
+//     256 units): 5.4 + 0.022 M per token (Q8_0 past K 4096 0.032), K-quants 6.2 +
+//     0.0225 M + 1.5e-5 N; tokens in fours, few rows longer (a round of
+//     blocks is not full): times 1 + 256 / N;
+//   Q5_0, Q4_1 (quantized inside every block, one launch less): 3.3 + the larger of a
+//     chain of 0.21 per 1024 of K for each of up to eight tokens of a block and
+//     M t times 0.03 (K to 512), 0.037 (2048), 0.066 (4096) or, past that, 0.08-0.2 by the
+//     tokens per block (their registers spill); the smaller adds 0.6 (0.3) of itself;
+//   rows of more than 256 units (blocks of 32: K > 8192, 64-groups: K > 16384), no
+//     pre-quantized form: 4 + 0.2 M t, up to 3 tokens 5 + 0.1 M t;
+//   Q6_K: 5 + 0.05 M t (K to 2048 0.038, 1024 0.07, 512 0.13: passes over super-blocks part filled);
+//   this form: its chain over K, 1.17 (K-quants), 1.55, 1.45 (Q8_0), 1.65 (Q5_0, Q4_1), 2.5 (Q6_K) per
+//     1024 of K, or its arithmetic per tile, 0.18 M + 1e-4 N, 0.215 M, 0.43 M + 3e-4 N
+//     (Q6_K), whichever is larger, and 5.2-5.6; at least 7 (Q6_K 8.2).
+// Measured, decode kernels / this form: Q4_K 14336x4096 at 8 / 16 / 32 / 64
+// tokens 19.2 / 28.3 / 47.2 / 87.0 against 18.3 / 18.4 / 25.9 / 44.1; Q4_0 4096x14336 at
+// 4 / 16 / 64 54 / 194 / 768 against 28 / 28 / 48; Q5_0 4096x512 at 4 / 32 4.1 /
+// 5.3 against 6.9 / 6.9, 4096x4096 at 4 / 16 8.6 / 23.4 against 12.0 / 12.1; Q6_K 2048x5632
+// at 8 / 24 / 32 11.5 / 18.5 / 22.0 against 20.2 / 20.6 / 20.6.  Of the
+// 3528 shapes timed, the form taken is within 10 % of the faster one at 3489 (with one set of
+// decode costs for all formats 3077: Q5_0 and Q4_1 came here at short K, 4.1 -> 7.0 us).
 // RCE_QMM_Q8_MFMA: 0 = never this form, 2 = always where it applies (tests of
 // both forms on the same shapes).  Read at every call, so a test can switch it.
 bool gemv_q8_mfma_preferred(const DevWeight &w, size_t t_rows) {
     const char *e = getenv("RCE_QMM_Q8_MFMA");
     const int mode = e ? atoi(e) : 1;
     if (mode != 1) return mode == 2;
-    const double m = (double)w.n_rows * (double)w.n_cols * 1e-6, t = (double)t_rows, k = (double)w.n_cols / 1024.0;
+    const size_t K = w.n_cols;
+    const double n = (double)w.n_rows, m = n * (double)K * 1e-6, t = (double)t_rows, k = (double)K / 1024.0;
+    const double t4 = t_rows < 4 ? t : (double)((t_rows + 3) / 4 * 4), tiles = (double)((t_rows + 15) / 16);
     const bool q6 = w.dtype == T_Q6_K, kq = w.dtype == T_Q4_K || w.dtype == T_Q5_K;
-    const double decode = q6 ? 5.0 + 0.05 * m * t
-                             : nt_for(units_per_row(w.dtype, w.n_cols)) != 256 && t_rows >= 4 ? 4.0 + 0.2 * m * t
-                                                                                            : 7.3 + 0.021 * m * t;
-    const double chain = (q6 ? 2.7 : kq ? 1.2 : 1.6) * k, work = (q6 ? 0.43 : 0.18) * m * (double)((t_rows + 15) / 16);
-    return 5.0 + (chain > work ? chain : work) < decode;
+    const bool inl = w.dtype == T_Q5_0 || w.dtype == T_Q4_1;
+    double decode, self;
+    if (q6) {
+        decode = 5.0 + (K <= 512 ? 0.13 : K <= 1024 ? 0.07 : K <= 2048 ? 0.038 : 0.05) * m * t;
+        self = std::max(8.2, 5.6 + std::max(2.5 * k, (0.43 * m + 3e-4 * n) * tiles));
+    } else if (kq) {
+        decode = std::max(t_rows < 4 ? 6.3 : 7.1, 6.2 + (0.0225 * m + 1.5e-5 * n) * t4 * (1.0 + 256.0 / n));
+        self = std::max(7.0, 5.2 + std::max(1.17 * k, (0.18 * m + 1e-4 * n) * tiles));
+    } else {
+        const double chain = 0.21 * k * std::min(t, 8.0);
+        const double slope = K <= 512 ? 0.03 : K <= 2048 ? 0.037 : K <= 4096 ? 0.066 : t_rows >= 8 ? 0.2 : t_rows >= 4 ? 0.13 : 0.08;
+        if (inl) decode = 3.3 + std::max(chain, slope * m * t) + (K <= 2048 ? 0.6 : K <= 4096 ? 0.3 : 0.0) * std::min(chain, slope * m * t);
+        else decode = std::max(6.4, 5.4 + (w.dtype == T_Q8_0 && K > 4096 ? 0.032 : 0.022) * m * t4 * (1.0 + 256.0 / n));
+        self = std::max(6.9, 5.6 + std::max((inl ? 1.65 : w.dtype == T_Q8_0 ? 1.45 : 1.55) * k, 0.215 * m * tiles));
+    }
+    if (!q6 && nt_for(units_per_row(w.dtype, K)) != 256) decode = t_rows >= 4 ? 4.0 + 0.2 * m * t : 5.0 + 0.1 * m * t;
+    return self < decode;
 }
 
 size_t gemv_q8_tile_bytes(size_t n_cols) { return n_cols / QK * ACT_STAGE; }

@@ -11,6 +11,7 @@ import rce_amd
 from rand_blocks import rand_blocks
 from rce_amd import Mode
 from rce_amd._lib import check, lib
+from test_gpu_gemm_wide import weight_bytes
 from test_gpu_gemv import bits, run_dev
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +61,23 @@ def test_outputs_past_the_grid_limit(ctx, monkeypatch):
         check(lib().rce_qmm_memcpy_d2h(ctx.handle, ctypes.c_void_p(got.ctypes.data), ctypes.c_void_p(out.ptr + 4 * n * t0), got.nbytes))
         assert np.array_equal(bits(got), bits(run_dev(ctx, w, x[t0:t0 + 4], Mode.Q8))), t0
     xa.free(); out.free(); w.close()
+
+
+@pytest.mark.parametrize("dt", FORMATS)
+@pytest.mark.parametrize("n,k,t", [(40, 512, 2), (40, 512, 48), (72, 4096, 13), (1030, 2048, 24), (24, 16640, 5)])
+def test_the_rule_changes_no_bits(ctx, monkeypatch, dt, n, k, t):
+    """The form the rule takes on both sides of its lines (short and long
+    rows, rows of more than 256 units, few and many tokens), and either form forced."""
+    print(f"q8 rule dtype={dt} n={n} k={k} t={t}", flush=True)
+    rng = np.random.default_rng(dt * 1000 + n + t)
+    w = rce_amd.QuantWeight.from_owned_bytes(ctx, weight_bytes(rng, dt, n, k), dt, n, k)
+    x = rng.standard_normal((t, k)).astype(np.float32)
+    got = []
+    for form in (None, "0", "2"):
+        if form is None:
+            monkeypatch.delenv("RCE_QMM_Q8_MFMA", raising=False)
+        else:
+            monkeypatch.setenv("RCE_QMM_Q8_MFMA", form)
+        got.append(bits(run_dev(ctx, w, x, Mode.Q8)))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    w.close()
