@@ -37,6 +37,8 @@
 #include "mfma_util.h"
 #include "qmm_internal.h"
 
+#include <algorithm>
+
 namespace rce_qmm {
 namespace {
 
@@ -671,44 +673,66 @@ double wide_rounds(size_t tiles, size_t cus, double full, double lo) {
     return (double)r * full + (m == 0 ? 0.0 : m <= knee ? lo : lo + (full - lo) * (double)(m - knee) / (double)(cus - knee));
 }
 
+// Microseconds of one round of tiles at K 4096 on 256 CUs, {every CU busy, at
+// most half of them}: 128 x 128, 128 x 256, 256 x 128 and 256 x 256 here, 128 x 64
+// and (a full round) 96 x 128 in gemm_f16.hip.  Fitted to every shape of every format
+// at M 128-2048, N 1024-14336.  Fifth bits cost a multiply per four weights in each
+// of the waves that share a column, Q6_K's two bit planes less.
+struct WideCost {
+    double t128[2], t128x256[2], t256x128[2], t256[2], t128x64[2], t96x128;
+};
+const WideCost &wide_cost(uint32_t dtype) {
+    static const WideCost plain = {{46.5, 38.0}, {79.0, 60.0}, {72.0, 52.0}, {126.0, 83.0}, {25.0, 19.0}, 34.5};
+    static const WideCost fifth = {{52.0, 45.0}, {86.0, 72.0}, {73.5, 57.0}, {132.5, 96.0}, {25.0, 18.0}, 35.0};
+    static const WideCost q6 = {{46.5, 40.5}, {81.0, 69.0}, {69.0, 49.5}, {126.0, 88.5}, {24.0, 18.0}, 0.0};
+    return dtype == T_Q5_K || dtype == T_Q5_0 ? fifth : dtype == T_Q6_K ? q6 : plain;
+}
+
+// The estimated time of gemm_f16.hip's tiles.  Its last row tile runs a 64- or
+// 96-row body where it holds no more rows; a round there has a fixed part
+// (measured against the tiles here: +24 % at K 1024, -6 % at K 14336).
+double small_tile_cost(const DevWeight &w, size_t M, size_t cus, const WideCost &c) {
+    const size_t N = w.n_rows, n64 = (N + 63) / 64, t = (M + 127) / 128 * n64, rounds = (t + cus - 1) / cus, rem = M % 128;
+    double v = wide_rounds(t, cus, c.t128x64[0], c.t128x64[1]);
+    if (rounds > 1 && rem > 0 && rem <= 96 && n64 >= t - (rounds - 1) * cus) v -= (rem <= 64 ? 0.45 : 0.2) * c.t128x64[0];
+    if (w.dtype != T_Q8_0 && w.dtype != T_Q6_K)
+        v = std::min(v, c.t96x128 * (double)(((M + 95) / 96 * ((N + 127) / 128) + cus - 1) / cus));
+    return v * (0.92 + 0.08 * 4096.0 / (double)w.n_cols);
+}
+
 // The tile shape for out[M, N], or WIDE_NONE where gemm_f16.hip's tiles are
-// estimated faster.  The constants are microseconds measured at K 4096
-// (Q4_K; every shape scales alike with K) on 256 CUs, full round / at most
-// half of the CUs busy: 256 x 256 126 / 83, 128 x 256 79 / 57.5, 256 x 128
-// 72 / 52, 128 x 128 46.5 / 37.5; the 128 x 64 tile 25 per round and the
-// 96 x 128 tile 34.5.  Per 128 x 128 outputs that is 31, 40, 36, 46 and 50,
-// so the larger tiles win as soon as they fill the chip: M 1024 x N 4096
-// 50 -> 47 us on 128 x 128, M 2048 x N 4096 103 -> 75 on 256 x 128, M 4096 x
-// N 14336 1070 -> 447 on 256 x 256 with the last half round as 128 x 256.
+// estimated faster.  Per 128 x 128 outputs a plain format's full round is 31 us in
+// 256 x 256 tiles, 36 in 256 x 128, 40 in 128 x 256, 46 in 128 x 128 and 50 in 128 x 64, so
+// the larger tiles win as soon as they fill the chip: M 1024 x N 4096 50 -> 47
+// us on 128 x 128, M 2048 x N 4096 103 -> 75 on 256 x 128, M 4096 x N 14336
+// 1070 -> 447 on 256 x 256 with the last half round as 128 x 256.  With one
+// set of costs for all formats, Q5_K, Q5_0 and Q6_K came here where the small
+// tiles are faster: Q5_K M 200 x N 14336 at K 14336 131 us there, 176 here.
 // F16 weights always come here (K 2560, M 333, N 6912: 45 us in
 // gemm_gen.hip, 20 here; M 16, N 2048: 21 / 15).
 WideShape wide_shape(const DevWeight &w, size_t M, size_t cus) {
     const size_t N = w.n_rows;
     auto tiles = [&](size_t bm, size_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    const bool f16 = w.dtype == T_F16;
     WideShape best = WIDE_NONE;
     double cost = 0.0;
     auto offer = [&](WideShape sh, double c) {
         if (best == WIDE_NONE ? (cost == 0.0 || c < cost) : c < cost) { best = sh; cost = c; }
     };
-    if (f16) {
+    if (w.dtype == T_F16) {
         offer(WIDE_128x128, wide_rounds(tiles(128, 128), cus, 22.0, 15.5));
         offer(WIDE_128x256, wide_rounds(tiles(128, 256), cus, 43.0, 25.0));
         offer(WIDE_256x128, wide_rounds(tiles(256, 128), cus, 43.5, 26.0));
         return best;
     }
-    cost = 25.0 * (double)((tiles(128, 64) + cus - 1) / cus);
-    if (w.dtype != T_Q8_0 && w.dtype != T_Q6_K) {
-        const double c96 = 34.5 * (double)((tiles(96, 128) + cus - 1) / cus);
-        cost = c96 < cost ? c96 : cost;
-    }
-    offer(WIDE_128x128, wide_rounds(tiles(128, 128), cus, 46.5, 37.5));
-    offer(WIDE_128x256, wide_rounds(tiles(128, 256), cus, 79.0, 57.5));
-    offer(WIDE_256x128, wide_rounds(tiles(256, 128), cus, 72.0, 52.0));
+    const WideCost &c = wide_cost(w.dtype);
+    cost = small_tile_cost(w, M, cus, c);
+    offer(WIDE_128x128, wide_rounds(tiles(128, 128), cus, c.t128[0], c.t128[1]));
+    offer(WIDE_128x256, wide_rounds(tiles(128, 256), cus, c.t128x256[0], c.t128x256[1]));
+    offer(WIDE_256x128, wide_rounds(tiles(256, 128), cus, c.t256x128[0], c.t256x128[1]));
     const size_t t = tiles(256, 256), rem = t % cus;
-    offer(WIDE_256x256, wide_rounds(t, cus, 126.0, 83.0));
+    offer(WIDE_256x256, wide_rounds(t, cus, c.t256[0], c.t256[1]));
     if (t > cus && rem && 2 * rem <= cus)
-        offer(WIDE_256x256_TAIL, (double)(t / cus) * 126.0 + wide_rounds(2 * rem, cus, 79.0, 57.5));
+        offer(WIDE_256x256_TAIL, (double)(t / cus) * c.t256[0] + wide_rounds(2 * rem, cus, c.t128x256[0], c.t128x256[1]));
     return best;
 }
 

@@ -23,7 +23,7 @@ F16, F32 = np.float16, np.float32
 QUANT = [O.Q4_K, O.Q5_K, O.Q4_0, O.Q4_1, O.Q5_0, O.Q8_0, O.Q6_K]
 # (tokens, rows): one case per tile shape on a 256-CU chip
 SHAPES = {"128x128": (1000, 4000), "256x128": (2000, 4040), "128x256": (600, 11000), "256x256": (1000, 11000),
-          "256x256 then 128x256": (1500, 11000)}
+          "256x256 then 128x256": (3000, 11000)}
 
 
 def weight_bytes(rng, dt, n, k):
@@ -32,10 +32,13 @@ def weight_bytes(rng, dt, n, k):
     return rce_amd.quantize((rng.standard_normal((n, k)) * 0.02).astype(F32), dt)
 
 
+# K: one super-block (two weight stages, none loaded into a slot twice), and
+# an odd number of them (every slot of the rings refilled)
+@pytest.mark.parametrize("k", [256, 768])
 @pytest.mark.parametrize("dt", QUANT)
 @pytest.mark.parametrize("shape", sorted(SHAPES))
-def test_wide_tiles_match_the_small_tile_kernel(ctx, dt, shape):
-    (m, n), k = SHAPES[shape], 256 if dt % 2 else 768  # one super-block, and an odd number of them
+def test_wide_tiles_match_the_small_tile_kernel(ctx, dt, shape, k):
+    m, n = SHAPES[shape]
     print(f"wide tile {shape} dtype={dt} M={m} N={n} K={k}", flush=True)
     rng = np.random.default_rng(dt)
     w = rce_amd.QuantWeight.from_owned_bytes(ctx, weight_bytes(rng, dt, n, k), dt, n, k)
