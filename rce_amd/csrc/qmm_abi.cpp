@@ -570,6 +570,29 @@ bool moe_q8_mfma_preferred(double rows_per_expert, bool q6, bool by_tile) {
     return !by_tile || rows_per_expert >= (q6 ? 8.0 : 4.0);
 }
 
+// EXACT grouped experts: all in one launch over tiles of one and two slots, or
+// one product per expert, which waits for the grouping on the host and makes
+// launches for every expert but, with many slots, uses the decode kernels'
+// shapes of up to 16 rows per lane.  `m` is the multiply-adds of the call in 10^6.  Fitted
+// to 4 and 8 experts top-1 and top-2 of 1024x2816, 2048x5632 and 4096x14336 at 16-256 tokens: the
+// launches and the wait cost 40 us and 10 per expert; the tiles cost more per
+// 10^6 by 0.018 us (Q8_0, Q4_1, Q5_K), 0.010 (Q4_K), 0.007 (Q4_0, Q5_0, Q3_K), nothing (Q6_K, one
+// kernel for both).  One product per expert / tiles (us), 8 experts top-2, 2048x5632 at 64
+// and 256 tokens: Q8_0 460 / 373, 1241 / 1361; Q5_K 1426 / 1527 at 256; Q4_0 518 / 371, 1428 /
+// 1327; 4096x14336 at 16, 64 and 256: Q8_0 595 / 544, 1721 / 1764, 6126 / 6821; Q4_0 634 / 487, 1685 /
+// 1597, 5917 / 6194; Q6_K 20542 / 20421 at 256.
+bool moe_exact_tiles_preferred(uint32_t t1, uint32_t t2, size_t n_expert, double m1, double m2) {
+    auto extra = [](uint32_t t) {
+        switch (t) {
+        case T_Q6_K: return 0.0;
+        case T_Q4_0: case T_Q5_0: case T_Q3_K: return 0.007;
+        case T_Q4_K: return 0.010;
+        default: return 0.018;
+        }
+    };
+    return extra(t1) * m1 + extra(t2) * m2 < 40.0 + 10.0 * (double)n_expert;
+}
+
 // The grouped experts: h = silu(W1 x) (w3 == nullptr, the benchmark's
 // two-matrix expert) or h = silu(W1 x) * (W3 x) (SwiGLU: W1 = gate, W3 =
 // up), y = W2 h, out = the decision-order combine.
@@ -633,6 +656,8 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
         const bool args = n_expert <= MOE_ARG_EXPERTS && n_pairs + n_expert <= 65535;
         if (args && gemv_grouped_supports(a1.dtype, d_model, (int)mode) && gemv_grouped_supports(a2.dtype, d_ff, (int)mode))
             form = BY_TILE;
+        const double m = (double)n_pairs * (double)d_model * (double)d_ff * 1e-6;
+        if (mode == RCE_QMM_MODE_EXACT && !moe_exact_tiles_preferred(a1.dtype, a2.dtype, n_expert, w3 ? 2.0 * m : m, m)) form = BY_EXPERT;
         const size_t tiles16 = n_pairs / 16 + n_expert;
         if (args && mode == RCE_QMM_MODE_Q8 && gemv_q8_grouped_supports(a1, tiles16) && gemv_q8_grouped_supports(a2, tiles16) &&
             moe_q8_mfma_preferred(per_expert, a1.dtype == T_Q6_K || a2.dtype == T_Q6_K, form != BY_EXPERT))

@@ -92,3 +92,16 @@ def test_many_experts_expert_by_expert_q8(ctx, monkeypatch, mma):
     gw = np.full((t, 2), 0.5, np.float32)
     got = run_moe(ctx, w1, w2, O.Q4_0, dm, dff, x, ids, gw, Mode.Q8)
     assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q4_0, dff, ids, gw, q8=True, silu_dev=True))
+
+
+@pytest.mark.parametrize("t", [1300, 1340])
+def test_exact_forms_on_both_sides_of_the_rule(ctx, t):
+    """One Q8_0 expert of 512 x 2048: 2726 and 2810 million multiply-adds, in tiles
+    of two slots and as a product of its own."""
+    print(f"moe exact rule t={t}", flush=True)
+    rng = np.random.default_rng(t)
+    w1, w2 = experts(rng, O.Q8_0, 1, 2048, 512), experts(rng, O.Q8_0, 1, 512, 2048)
+    x = rng.standard_normal((t, 512)).astype(np.float32)
+    ids, gw = np.zeros((t, 1), np.int32), np.ones((t, 1), np.float32)
+    got = run_moe(ctx, w1, w2, O.Q8_0, 512, 2048, x, ids, gw, Mode.EXACT)
+    assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q8_0, 2048, ids, gw, silu_dev=True))
