@@ -225,7 +225,8 @@ __global__ void k_swiglu_slots(float *__restrict__ g, const float *__restrict__ 
 // a thread's loads of y are one float4 per decision, all in flight at once.
 __global__ __launch_bounds__(256) void k_moe_combine4(const float *__restrict__ y, const int *__restrict__ slot_of_pair,
                                                       const float *__restrict__ gate_w, int top_k, size_t d,
-                                                      float *__restrict__ out) {
+                                                      float *__restrict__ out, const int *__restrict__ status) {
+    if (status && status[0]) return;
     const size_t t = blockIdx.x, d4 = d / 4;
     const float4 *y4 = reinterpret_cast<const float4 *>(y);
     float4 *o4 = reinterpret_cast<float4 *>(out) + t * d4;
@@ -248,7 +249,8 @@ __global__ __launch_bounds__(256) void k_moe_combine4(const float *__restrict__ 
 
 __global__ void k_moe_combine(const float *__restrict__ y, const int *__restrict__ slot_of_pair,
                               const float *__restrict__ gate_w, int top_k, size_t t_rows, size_t d,
-                              float *__restrict__ out) {
+                              float *__restrict__ out, const int *__restrict__ status) {
+    if (status && status[0]) return;
     for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < t_rows * d; k += (size_t)gridDim.x * blockDim.x) {
         const size_t t = k / d, i = k - t * d;
         float acc = 0.0f;
@@ -302,16 +304,16 @@ hipError_t launch_swiglu_slots(float *g, const float *u, const int *n_slots_dev,
 }
 
 hipError_t launch_moe_combine(const float *y, const int *slot_of_pair, const float *gate_w, size_t t_rows, int top_k,
-                              size_t d, float *out, hipStream_t s) {
+                              size_t d, float *out, const int *status, hipStream_t s) {
     if (t_rows == 0) return hipSuccess;
     if (d % 4 == 0 && t_rows <= 0xFFFFFFFFu / 256) {  // grid.x * 256 threads within 32 bits
         const size_t cy = d >= 4 ? (d / 4 + 255) / 256 : 1;
         hipLaunchKernelGGL(k_moe_combine4, dim3((unsigned)t_rows, (unsigned)(cy < 65535 ? cy : 65535)), dim3(256), 0, s, y,
-                           slot_of_pair, gate_w, top_k, d, out);
+                           slot_of_pair, gate_w, top_k, d, out, status);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_moe_combine, dim3(grid_1d(t_rows * d, 256)), dim3(256), 0, s, y, slot_of_pair, gate_w, top_k,
-                       t_rows, d, out);
+                       t_rows, d, out, status);
     return hipGetLastError();
 }
 

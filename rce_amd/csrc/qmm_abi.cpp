@@ -791,7 +791,8 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
             m.out2 = nullptr;
             HIP_TRY(launch_gemv_grouped(a2, m, q8 ? q : h, y, (int)mode, s));
         }
-        HIP_TRY(launch_moe_combine(y, slot_of_pair, weights_dev, t_rows, (int)top_k, d_model, out_dev, s));
+        // (an id out of range leaves out_dev as it is)
+        HIP_TRY(launch_moe_combine(y, slot_of_pair, weights_dev, t_rows, (int)top_k, d_model, out_dev, status, s));
         HIP_TRY(hipEventSynchronize(ctx->moe_grouped));
         if (*static_cast<volatile int *>(ctx->moe_status)) return fail(RCE_QMM_BAD_SHAPE, "an expert id is out of range");
         return RCE_QMM_OK;
@@ -849,7 +850,7 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
         }
     }
     // 5. combine in decision order
-    HIP_TRY(launch_moe_combine(y, slot_of_pair, weights_dev, t_rows, (int)top_k, d_model, out_dev, s));
+    HIP_TRY(launch_moe_combine(y, slot_of_pair, weights_dev, t_rows, (int)top_k, d_model, out_dev, nullptr, s));
     return RCE_QMM_OK;
 }
 

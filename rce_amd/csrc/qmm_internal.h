@@ -497,9 +497,10 @@ hipError_t launch_silu_inplace(float *h, const int *n_slots_dev, size_t max_slot
 // in place.
 hipError_t launch_swiglu_slots(float *g, const float *u, const int *n_slots_dev, size_t max_slots, size_t d,
                                hipStream_t s);
-// out[t, :] = sum_j gate_w[t, j] * y[slot_of_pair[t * top_k + j], :], j in order, from +0.0
+// out[t, :] = sum_j gate_w[t, j] * y[slot_of_pair[t * top_k + j], :], j in order, from +0.0;
+// nothing where status (launch_moe_group's, may be null) is set
 hipError_t launch_moe_combine(const float *y, const int *slot_of_pair, const float *gate_w, size_t t_rows, int top_k,
-                              size_t d, float *out, hipStream_t s);
+                              size_t d, float *out, const int *status, hipStream_t s);
 // What the grouped GEMM stores for output element o with f32 sum v:
 // v (f32 out), binary16 silu(v), or binary16 silu(aux[o]) * v (aux: the
 // f32 gate products of the same slots, SwiGLU).

@@ -105,3 +105,24 @@ def test_exact_forms_on_both_sides_of_the_rule(ctx, t):
     ids, gw = np.zeros((t, 1), np.int32), np.ones((t, 1), np.float32)
     got = run_moe(ctx, w1, w2, O.Q8_0, 512, 2048, x, ids, gw, Mode.EXACT)
     assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q8_0, 2048, ids, gw, silu_dev=True))
+
+
+@pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
+@pytest.mark.parametrize("E,dm", [(4, 256), (65, 256)])  # the grouped forms; expert by expert
+def test_bad_id_leaves_the_output(ctx, mode, E, dm):
+    print(f"bad id E={E} mode={mode}", flush=True)
+    rng = np.random.default_rng(4)
+    W1 = [rce_amd.QuantWeight.from_owned_bytes(ctx, b, O.Q4_0, 512, dm) for b in experts(rng, O.Q4_0, E, 512, dm)]
+    W2 = [rce_amd.QuantWeight.from_owned_bytes(ctx, b, O.Q4_0, dm, 512) for b in experts(rng, O.Q4_0, E, dm, 512)]
+    ids = np.array([[0, 1], [2, E]], np.int32)
+    keep = rng.standard_normal(2 * dm).astype(np.float32)
+    bufs = [rce_amd.DeviceBuffer.from_numpy(ctx, a) for a in (rng.standard_normal((2, dm)).astype(np.float32), ids,
+                                                             np.full((2, 2), 0.5, np.float32), keep)]
+    with pytest.raises(rce_amd.QmmError, match="out of range"):
+        rce_amd.moe_ffn_dev(ctx, W1, W2, bufs[0].ptr, 2, bufs[1].ptr, bufs[2].ptr, 2, bufs[3].ptr, mode)
+    ctx.synchronize()
+    assert np.array_equal(bufs[3].download(np.float32, 2 * dm), keep)
+    for x in bufs:
+        x.free()
+    for w in W1 + W2:
+        w.close()
