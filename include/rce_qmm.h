@@ -221,8 +221,10 @@ rce_qmm_status rce_qmm_mm_batched_dev(rce_qmm_context *ctx, const void *a_dev, u
  * kernels and bits, and no hipMalloc / hipFree / allocating library call.
  * The scratch the call needs -- 4 t_rows n_cols bytes to widen F16
  * activations (EXACT, Q8), 1.375 t_rows n_cols bytes for several tokens'
- * Q8 activations (Q8, t_rows >= 2), 2 t_rows n_cols bytes to round F32
- * activations to f16 (F16_MFMA), each rounded up to 256 -- comes from a
+ * Q8 activations (Q8, t_rows >= 2: Q4_0 / Q8_0 with n_cols a multiple of
+ * 256 or at most 8192, Q4_K / Q5_K up to 16384 columns, Q6_K), 2
+ * t_rows n_cols bytes to round F32 activations to f16 (F16_MFMA), each
+ * rounded up to 256 and counted by dtype and shape alone -- comes from a
  * fixed device array of RCE_QMM_NOALLOC_SCRATCH_BYTES that each GPU the
  * library runs on holds until the process ends; a call that needs more
  * returns RCE_QMM_BAD_SHAPE.  All calls on one GPU share that array:

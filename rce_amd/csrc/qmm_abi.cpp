@@ -72,16 +72,28 @@ struct BatchedScratch {
 
 }  // namespace
 
-// The scratch bytes mm_batched_dev needs for these arguments (the parts
-// BatchedScratch names, each rounded up to 256 bytes), given a supported
-// (dtype, n_cols, mode).
+// Whether several tokens' Q8 activations count towards the fixed scratch: by
+// format and shape alone, whichever form a call takes, so that what the
+// no-allocation entry refuses does not move with the dispatch.
+static bool q8_counted(uint32_t dtype, size_t k, size_t t_rows) {
+    if (t_rows < 2 || t_rows > 65535 * 8 || !gpu_supports(dtype, k, 1)) return false;
+    const bool narrow = k <= (dtype == T_Q4_0 || dtype == T_Q8_0 ? 8192 : dtype == T_Q6_K ? 65536 : 16384);  // at most 256 units
+    switch (dtype) {
+    case T_Q4_0: case T_Q8_0: return narrow || (k % 256 == 0 && t_rows * (k / 8) < ((size_t)1 << 31));
+    case T_Q4_K: case T_Q5_K: case T_Q6_K: return narrow;
+    default: return false;
+    }
+}
+
+// The scratch bytes a no-allocation call counts for these arguments, each
+// part rounded up to 256 bytes, given a supported (dtype, n_cols, mode).
 size_t rce_qmm_abi::batched_scratch_bytes(const DevWeight &dw, uint32_t a_dtype, size_t t_rows, rce_qmm_mode mode) {
     const size_t k = dw.n_cols;
     if (t_rows == 0 || dw.n_rows == 0) return 0;
     if (mode == RCE_QMM_MODE_F16_MFMA) return a_dtype == T_F16 ? 0 : align_up(t_rows * k * 2, 256);
     size_t b = 0;
     if (a_dtype == T_F16) b += align_up(t_rows * k * sizeof(float), 256);
-    if (mode == RCE_QMM_MODE_Q8 && gemv_q8_pre_supports(dw.dtype, k, t_rows)) b += align_up(t_rows * (k + k / 8 + k / 4), 256);
+    if (mode == RCE_QMM_MODE_Q8 && q8_counted(dw.dtype, k, t_rows)) b += align_up(t_rows * (k + k / 8 + k / 4), 256);
     return b;
 }
 
@@ -148,6 +160,12 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     const size_t k = dw.n_cols;
     const bool mfma = mode == RCE_QMM_MODE_F16_MFMA;
     const bool widen = !mfma && a_dtype == T_F16;
+    if (fixed) {
+        const size_t need = batched_scratch_bytes(dw, a_dtype, t_rows, mode);
+        if (need > fixed_cap)
+            return fail(RCE_QMM_BAD_SHAPE, "the call needs " + std::to_string(need) + " bytes of scratch; the fixed scratch holds " +
+                                               std::to_string(fixed_cap));
+    }
     const bool preq = mode == RCE_QMM_MODE_Q8 && gemv_q8_pre_supports(dw.dtype, k, t_rows);
     const size_t f32_b = widen ? t_rows * k * sizeof(float) : 0;
     size_t q8_b = preq ? t_rows * (k + k / 8 + k / 4) : 0;  // xq, dx, s16
@@ -166,10 +184,6 @@ rce_qmm_status rce_qmm_abi::run_batched(rce_qmm_context *ctx, const void *a_dev,
     BatchedScratch sc;
     rce_qmm_status st;
     if (fixed) {
-        const size_t need = batched_scratch_bytes(dw, a_dtype, t_rows, mode);
-        if (!mma && need > fixed_cap)
-            return fail(RCE_QMM_BAD_SHAPE, "the call needs " + std::to_string(need) + " bytes of scratch; the fixed scratch holds " +
-                                               std::to_string(fixed_cap));
         unsigned char *p = static_cast<unsigned char *>(fixed);
         if (f32_b) { sc.a_f32 = reinterpret_cast<float *>(p); p += align_up(f32_b, 256); }
         if (q8_b) { sc.act_q = p; p += align_up(q8_b, 256); }

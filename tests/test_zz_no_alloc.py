@@ -83,3 +83,25 @@ def test_noalloc_rejects_scratch_beyond_the_fixed_array(ctx):
     rce_amd.mm_batched_dev_noalloc(ctx, xa.ptr, G.F32, 0, qw, out.ptr, Mode.Q8)
     ctx.synchronize()
     xa.free(); out.free(); qw.close()
+
+
+@pytest.mark.parametrize("dt,k,t", [(O.Q4_0, 16384, 800), (O.Q8_0, 14336, 860), (O.Q4_K, 14336, 860), (O.Q6_K, 14336, 860)])
+def test_noalloc_counts_the_documented_bytes(ctx, dt, k, t):
+    """1.375 t k bytes past the fixed array are refused whichever kernel would
+    run (the matrix-core form's tiles are 1.25 t k and fit); the most tokens
+    within it are accepted."""
+    cap = rce_amd.NOALLOC_SCRATCH_BYTES
+    assert t * k * 11 // 8 > cap >= (t + 15) // 16 * 16 * k * 5 // 4
+    note(f"noalloc bytes dtype={dt} k={k} t={t}")
+    rng = np.random.default_rng(dt)
+    n = 32
+    qw = rce_amd.QuantWeight.from_owned_bytes(ctx, O.quantize((rng.standard_normal((n, k)) * 0.02).astype(F32), dt), dt, n, k)
+    a = rng.standard_normal((t, k)).astype(F32)
+    xa, out = rce_amd.DeviceBuffer.from_numpy(ctx, a), rce_amd.DeviceBuffer(ctx, 4 * t * n)
+    with pytest.raises(rce_amd.QmmError) as e:
+        rce_amd.mm_batched_dev_noalloc(ctx, xa.ptr, G.F32, t, qw, out.ptr, Mode.Q8)
+    assert e.value.status == 2 and "scratch" in str(e.value)
+    fits = cap * 8 // 11 // k
+    want, got = run_pair(ctx, qw, a[:fits], G.F32, fits, n, Mode.Q8)
+    assert not np.isnan(want).any() and np.array_equal(want.view(np.uint32), got.view(np.uint32))
+    xa.free(); out.free(); qw.close()
