@@ -748,7 +748,7 @@ hipError_t launch_gemv_fx(const FxLaunch &f, const float *a, int mode, hipStream
 
 bool gemv_q8_pre_supports(uint32_t dtype, size_t n_cols, size_t t_rows) {
     if (t_rows < 2 || t_rows > 65535 * 8 || !gpu_supports(dtype, n_cols, 1)) return false;
-    if (dtype != T_Q4_0 && dtype != T_Q8_0 && dtype != T_Q4_K && dtype != T_Q5_K && dtype != T_Q6_K) return false;
+    if (dtype != T_Q4_0 && dtype != T_Q8_0 && dtype != T_Q4_K && dtype != T_Q5_K) return false;
     return nt_for(units_per_row(dtype, n_cols)) == 256;
 }
 
@@ -756,7 +756,6 @@ hipError_t launch_gemv_q8_pre(const DevWeight &w, const float *a, size_t t_rows,
                               hipStream_t s) {
     if (t_rows == 0 || w.n_rows == 0) return hipSuccess;
     if (!gemv_q8_pre_supports(w.dtype, w.n_cols, t_rows)) return launch_gemv(w, a, t_rows, out, 1, s);
-    if (w.dtype == T_Q6_K) return launch_gemv(w, a, t_rows, out, 1, s);  // its blocks quantize their two tokens
     GemvGeom g = pick_gemv_geom(w, t_rows, 1);
     if (g.nt != 256 || g.tb < 2) return launch_gemv(w, a, t_rows, out, 1, s);
     if (g.tb > 4) g.tb = 4;  // more token groups re-read the weight, mostly from the Infinity Cache

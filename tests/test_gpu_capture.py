@@ -66,7 +66,7 @@ def test_k_slices(record):
 
 
 @pytest.mark.parametrize("record", ["cold", "warm"])
-@pytest.mark.parametrize("dt", [O.Q5_0, O.Q4_1])
+@pytest.mark.parametrize("dt", [O.Q5_0, O.Q4_1, O.Q6_K])
 def test_q8_formats_without_scratch(monkeypatch, dt, record):
     """32 tokens recorded for formats whose decode kernels quantize inside
     their blocks, 200 (a larger workspace of the matrix-core form) and new
