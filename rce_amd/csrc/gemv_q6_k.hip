@@ -415,11 +415,9 @@ bool q6_rows32(size_t n_rows, size_t k, int tb, size_t units) {
 template <int TB, int R, int FX>
 hipError_t launch_q6_q8(const DevWeight &w, const float *a, size_t t_rows, float *out, const GemvFx &fx, dim3 grid,
                         hipStream_t s) {
-    const size_t lds = q6_q8_lds(w.n_cols, TB, R);  // 16 rows, two tokens, the longest row (act_lds_bytes(k, 1) = LDS_MAX): 151 KB
-    if (lds > LDS_MAX) {
-        const hipError_t e = ensure_lds_limit((const void *)k_gemv_q8_q6k<TB, R, FX>, 160 * 1024);
-        if (e != hipSuccess) return e;
-    }
+    // 16 rows, two tokens, the longest row (act_lds_bytes(k, 1) = LDS_MAX): 151 KB
+    // (past 64 KB: q6_prepare_lds has raised the limit)
+    const size_t lds = q6_q8_lds(w.n_cols, TB, R);
     hipLaunchKernelGGL((k_gemv_q8_q6k<TB, R, FX>), grid, dim3(256), lds, s, w, a, out, (int)t_rows, fx);
     return hipGetLastError();
 }
@@ -500,8 +498,17 @@ hipError_t launch_q6_split(const DevWeight &w, const float *a, size_t t_rows, fl
 }  // namespace
 
 hipError_t q6_prepare_lds() {
-    const hipError_t e = ensure_lds_limit((const void *)k_gemv_exact_q6k_split<false>, 160 * 1024);
-    return e != hipSuccess ? e : ensure_lds_limit((const void *)k_gemv_exact_q6k_split<true>, 160 * 1024);
+    // Q8: the forms with 16 rows per block (with 32, q6_rows32 keeps to 64 KB;
+    // the normalizing forms' rows are short)
+    for (const void *fn : {(const void *)k_gemv_exact_q6k_split<false>, (const void *)k_gemv_exact_q6k_split<true>,
+                           (const void *)k_gemv_q8_q6k<1, 16, 0>, (const void *)k_gemv_q8_q6k<2, 16, 0>,
+                           (const void *)k_gemv_q8_q6k<1, 16, FX_GROUP>, (const void *)k_gemv_q8_q6k<2, 16, FX_GROUP>,
+                           (const void *)k_gemv_q8_q6k<1, 16, FX_SEG>, (const void *)k_gemv_q8_q6k<1, 16, FX_RESIDUAL>,
+                           (const void *)k_gemv_q8_q6k<1, 16, FX_SWIGLU>}) {
+        const hipError_t e = ensure_lds_limit(fn, 160 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_gemv_grouped_q6_k(const DevWeight &w, const MoeGroup &m, const void *a, float *out, int mode, hipStream_t s) {

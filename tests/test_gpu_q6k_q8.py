@@ -11,6 +11,7 @@ from llama_case import make_weights, tiny_cfg
 from rce_amd import Mode
 from test_gpu_gemv import bits, run_dev
 from test_gpu_llama import TOKENS, run_pair
+from test_gpu_moe_forms import check
 
 pytestmark = pytest.mark.gpu
 
@@ -36,7 +37,8 @@ def test_bit_identical(ctx, monkeypatch, n, k, t):
 
 
 @pytest.mark.parametrize("norm_kernel", [False, True])  # the forms with and without rms_norm inside
-@pytest.mark.parametrize("d_ff", [512, 4352])           # gate/up and residual: whole blocks; a second pass of 16
+# gate/up and residual: whole blocks; a second pass of 16; a residual row past 64 KB of LDS
+@pytest.mark.parametrize("d_ff", [512, 4352, 40448])
 def test_fused_forms(ctx, monkeypatch, d_ff, norm_kernel):
     """A decoder whose linears are all Q6_K: q|k|v in one launch, the residual
     and gate/up forms and the head that ends the step, bit for bit against the
@@ -46,3 +48,9 @@ def test_fused_forms(ctx, monkeypatch, d_ff, norm_kernel):
         monkeypatch.setenv("RCE_QMM_LLAMA_NORM_KERNEL", "1")
     W = make_weights(tiny_cfg(d_ff=d_ff), seed=41, lin_dtype=O.Q6_K, embd_dtype=O.Q6_K)
     run_pair(ctx, W, Mode.Q8, TOKENS[:4], 1e-3, separate_norms=norm_kernel).close()
+
+
+def test_grouped_past_64_kb(ctx, monkeypatch):
+    """Two slots per block of a 20480-long row: 65 KB of LDS."""
+    monkeypatch.setenv("RCE_QMM_Q8_MFMA", "0")
+    check(ctx, O.Q6_K, 2, 256, 20480, 3, 2, Mode.Q8)
