@@ -385,8 +385,9 @@ def test_gemm_activations_past_4gib_sliced(ctx):
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q4_0, O.Q8_0])
 def test_gemm_rows_independent_of_tile_shape(ctx, dt):
     """Each output's sum is formed the same way in every tile shape and body
-    (a wave's k-step partial over the chunks in order, the four partials
-    added in order), so a row's result does not depend on how many rows the
+    of gemm_f16.hip (a wave's k-step partial over the chunks in order, the four
+    partials added in order), so among calls that run there in one piece, not in
+    K slices or the large tiles, a row's result does not depend on how many rows the
     call has: M 40 and 64 (a 64-row tile, 64 columns wide), 80 (96 rows),
     200 (128 rows, then a 72-row tile in the 96-row body) and 512 against
     the same rows of one another, bit for bit."""

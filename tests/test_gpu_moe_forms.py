@@ -44,6 +44,7 @@ def test_formats(ctx, dt, E, t, k, mode):
 def test_q8_on_the_matrix_cores(ctx, monkeypatch, dt):
     monkeypatch.setenv("RCE_QMM_Q8_MFMA", "2")
     check(ctx, dt, 3, 512, 768, 37, 2, Mode.Q8)  # about 25 slots per expert: a full tile and a ragged one
+    check(ctx, dt, 2, 2304, 2560, 20, 1, Mode.Q8)  # rows past 2048: a slot of every ring loaded again
 
 
 @pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])

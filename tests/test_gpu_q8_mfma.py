@@ -1,6 +1,7 @@
 """GPU parity of the int8 matrix-core form of the Q8 mode (gemv_q8_mfma.hip),
 forced on every case: the same bits as the oracle's Q8 restatement, at the
-edges of its tiles (16 tokens, 64 rows, stages of 256 with a ring of three)."""
+edges of its blocks (16 rows, tiles of 16 tokens; four waves taking chunks of
+256 of K, 128 for blocks of 32, in turn, each through a ring of two or three)."""
 import ctypes
 
 import numpy as np
@@ -16,10 +17,12 @@ from test_gpu_gemv import bits, run_dev
 
 pytestmark = pytest.mark.gpu
 FORMATS = [O.Q4_0, O.Q8_0, O.Q5_0, O.Q4_1, O.Q4_K, O.Q5_K, O.Q6_K]
-# (rows, columns, tokens): one row and one stage; ragged rows (scalar and
-# vector stores) and tokens around one and two tiles; stage counts 1, 2, 3
-# and 7; a row slice per XCD and one more
-SHAPES = [(1, 256, 2), (63, 256, 15), (66, 512, 16), (130, 768, 17), (576, 1792, 33)]
+# (rows, columns, tokens): one row, fewer chunks than waves; ragged rows and
+# tokens around one and two tiles; a last round of one, two and three waves; a row slice
+# per XCD and more; 9, 17 and 22 chunks of 256, where every slot of a ring is
+# loaded again (from the 9th chunk on in a ring of two), up to twice
+SHAPES = [(1, 256, 2), (63, 256, 15), (66, 512, 16), (130, 768, 17), (576, 1792, 33), (50, 2304, 18), (35, 4352, 33),
+          (20, 5632, 17)]
 
 
 @pytest.mark.parametrize("dt", FORMATS)
