@@ -31,6 +31,9 @@
  *                          contracted on the matrix cores with f32
  *                          accumulation in a fixed order; within 2e-3
  *                          normwise of mm_batched (grouped experts: 3e-3).
+ *                          The order is fixed for a shape: a row's last bits
+ *                          can differ between calls of different t_rows
+ *                          (tile shapes, slices of a short call's K).
  * Every mode is run-to-run bit-identical: no floating-point atomics, fixed
  * reduction trees.
  *
@@ -207,7 +210,10 @@ rce_qmm_status rce_qmm_quantize(uint32_t dtype, const float *src, size_t n_rows,
  * the reference's callers do), out_dev [t_rows, n_rows] f32.  No host
  * synchronization; the library's scratch is owned by the context, so calls
  * on one context must not overlap on different streams (one context per
- * stream).  RCE_QMM_MODE_F16_MFMA (the prefill form) takes Q4_K / Q4_0 /
+ * stream).  That scratch grows on demand: a call recorded into a HIP graph
+ * that uses it (F16 activations in EXACT / Q8, Q8 with several tokens, F32
+ * activations in F16_MFMA) is valid only until a larger call; record the
+ * no-allocation form below instead.  RCE_QMM_MODE_F16_MFMA (the prefill form) takes Q4_K / Q4_0 /
  * Q5_K / Q6_K with n_cols a multiple of 256 and Q8_0 / Q5_0 / Q4_1 / F16 /
  * BF16 / F32 with n_cols a multiple of 64 (rce_qmm_supports); its F16
  * activations must be 16-byte aligned. */
@@ -254,7 +260,9 @@ rce_qmm_status rce_qmm_moe_router(const float *logits, size_t n_tokens, size_t n
  * Q4_K_M file's Q4_K gate with its Q6_K down).  x_dev [t_rows, d_model] f32, ids_dev [t_rows, top_k]
  * i32, weights_dev [t_rows, top_k] f32, out_dev [t_rows, d_model] f32.
  * Tokens are grouped per expert on the device (stable by expert, then
- * token, then decision). */
+ * token, then decision).  EXACT and Q8 wait on the host for the grouping: an
+ * id outside [0, n_expert) returns RCE_QMM_BAD_SHAPE with out_dev unchanged;
+ * F16_MFMA does not wait and leaves such a pair out of its token's sum. */
 rce_qmm_status rce_qmm_moe_ffn_dev(rce_qmm_context *ctx, const rce_qmm_weight *const *w1,
                                    const rce_qmm_weight *const *w2, size_t n_expert,
                                    const float *x_dev, size_t t_rows, const int32_t *ids_dev,

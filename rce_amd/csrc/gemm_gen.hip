@@ -56,7 +56,7 @@ static_assert(DEPTH % CPB == 0 && DEPTH >= 2 * CPB, "load ring");
 // Output tile 128 x 64.  This kernel is bound by its dequantization into
 // LDS, done once per row tile and weight, so the tallest tile is the
 // cheapest: a 64 x 128 tile (built and measured) dequantizes every weight
-// once per 64 rows and took the configs[3] workload with Q6_K experts from
+// once per 64 rows and took 8 Q6_K experts of 14336x4096, 256 tokens top-2, from
 // 668 to 829 us.
 constexpr int BM = 128, BN = 64;
 constexpr int A_TILE = BM * KC * 2;               // 16 KB

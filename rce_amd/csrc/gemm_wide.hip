@@ -5,16 +5,18 @@
 // v_mfma_f32_32x32x16_f16 (f32 accumulation).
 //
 // The 128 x 64 tile of gemm_f16.hip copies 18 KB into LDS per 64-wide chunk
-// for 256 MFMA cycles per SIMD, and the copy path (about 50 B/clk per CU)
-// needs more than that.  Here a 256 x 256 tile copies 41 KB (Q4_K) for 2048
-// MFMA cycles, 20 B/clk, so the matrix cores set the pace as soon as the
-// problem holds enough such tiles.
+// for 256 MFMA cycles per SIMD, 70 B/clk per CU, and waits for those copies.
+// Here a 256 x 256 tile copies 41 KB (Q4_K) for 2048 MFMA cycles, 20 B/clk.
+// Counted at 4096 x 14336 x 4096 (Q4_K, 463 us at the 1.6 GHz the chip holds):
+// the matrix cores busy 63 % of the cycles, 4.9 other vector instructions and
+// 1.1 LDS instructions per MFMA, LDS bank conflicts (the reads of raw weight bytes; A's
+// have none) 18 % of a CU's cycles, A and W read 6 times from HBM between the eight L2s.
 //
 // Work split.  Eight waves, 2 (M) x 4 (N): a wave owns RB x CB blocks of
 // 32 x 32 outputs (tile 64 RB x 128 CB) over all of K, one accumulator
 // chain per output (k-steps of 16 in order).  Each wave dequantizes the W
-// fragments it consumes (each weight twice per tile, once per M half: 3.5
-// packed instructions per MFMA at RB = 4) from the raw bytes in LDS, so no
+// fragments it consumes (each weight twice per tile, once per M half: four
+// vector instructions per MFMA at RB = 4) from the raw bytes in LDS, so no
 // binary16 W tile is written.
 //
 // Pipeline.  K runs in chunks of 64 (four k-steps).  A is staged NSA - 1

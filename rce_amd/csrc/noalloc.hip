@@ -4,7 +4,8 @@
 // as rce_qmm_mm_batched_dev; the scratch those need (F16 activations widened
 // to f32, several tokens' Q8 activations quantized once, F32 activations
 // rounded to f16 for the MFMA GEMM) lives in `scratch`, a fixed device array
-// that every GPU the library runs on holds until the process ends.
+// that every GPU the library runs on holds until the process ends (the sums
+// of the GEMM's K slices live in a buffer allocated with the context).
 //
 // In host code `scratch` names a host-side stand-in, not device memory: the
 // array's device address on each GPU is resolved once, with that GPU

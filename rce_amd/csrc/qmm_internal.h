@@ -418,7 +418,7 @@ hipError_t launch_f32_to_f16(const float *src, void *dst, size_t n, hipStream_t 
 //   [x P, (x + 1) P), P = ceil(V / 8): each expert's tiles run on one or two
 //   XCDs, whose L2 then holds that expert's activation rows (with the
 //   (nt, mt) order every XCD read every expert's rows: 1.4x the HBM bytes
-//   of the expert weights on configs[3], 1.1x with this one, at the same
+//   of 8 experts' weights at 14336x4096, 256 tokens top-2, 1.1x with this one, at the same
 //   speed), and blocks past V return at once.
 __host__ __device__ inline int grouped_grid(int m_tiles, int col_tiles) { return (m_tiles * col_tiles + 7) / 8 * 8; }
 #ifdef __HIPCC__
