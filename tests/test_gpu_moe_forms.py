@@ -53,6 +53,26 @@ def test_expert_table_limits(ctx, E, mode):
     check(ctx, O.Q4_0, E, 256, 256, 40, 3, mode)
 
 
+@pytest.mark.parametrize("E", [2, 64])
+def test_mfma_expert_tables(ctx, E):
+    """F16_MFMA: the same experts in another order, and with one more that no
+    token takes (64: a table uploaded instead of written by the grouping
+    launch), give the same bits, within the mode's 3e-3 of the EXACT result."""
+    print(f"moe mfma tables E={E}", flush=True)
+    rng = np.random.default_rng(E)
+    dm, dff, t = 256, 512, 50
+    w1, w2 = experts(rng, O.Q4_0, E + 1, dff, dm), experts(rng, O.Q4_0, E + 1, dm, dff)
+    x = rng.standard_normal((t, dm)).astype(np.float32)
+    ids, gw = rce_amd.moe_router(rng.standard_normal((t, E)).astype(np.float32), 2)
+    got = [run_moe(ctx, w1[:E], w2[:E], O.Q4_0, dm, dff, x, ids, gw, Mode.F16_MFMA),
+           run_moe(ctx, w1[:E][::-1], w2[:E][::-1], O.Q4_0, dm, dff, x, E - 1 - ids, gw, Mode.F16_MFMA),
+           run_moe(ctx, w1, w2, O.Q4_0, dm, dff, x, ids, gw, Mode.F16_MFMA)]
+    assert bit_equal(got[0], got[1]) and bit_equal(got[0], got[2])
+    want = O.moe_ffn(x, w1, w2, O.Q4_0, dff, ids, gw)
+    # binary16 activations, weights and h, 2^-11 each, f32 sums: the mode's budget for grouped experts
+    assert np.linalg.norm(got[0].astype(np.float64) - want) < 3e-3 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
 def test_experts_change_between_calls(ctx, mode):
     """Two expert sets alternately on one context (a model's layers)."""
