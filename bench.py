@@ -1,7 +1,7 @@
 """Benchmark of the GGUF quantized-matmul path on one MI355X.
 
-Headline (BASELINE.json metric "GEMV HBM GB/s & GEMM TFLOPS per quant
-format, % of MI355X roofline", configs[1]): Q4_0 decode GEMV, weight
+Headline ("GEMV HBM GB/s & GEMM TFLOPS per quant format, % of MI355X
+roofline"): Q4_0 decode GEMV, weight
 11008x4096 N(0,0.02) quantized to Q4_0, activation batch 1 of 4096 f32
 N(0,1), in the reference's own f32 order (EXACT mode, bit-identical to
 mm_1d; --mode q8 for the Q8-activation mode).  A step is one GEMV launch over device-resident
@@ -214,7 +214,7 @@ def settle(ctx, run, settle_s):
 
 
 def time_gemm(hip, ctx, dt, n, k, m, steps, warmup, seed, settle_s=0.2):
-    """configs[2]-style prefill GEMM in F16_MFMA mode: A [m, k] f16 resident,
+    """Prefill GEMM in F16_MFMA mode: A [m, k] f16 resident,
     weights rotated over HBM copies; returns ms per launch and the first 16
     output rows (checked in the CPU leg)."""
     import rce_amd
@@ -246,7 +246,7 @@ def time_gemm(hip, ctx, dt, n, k, m, steps, warmup, seed, settle_s=0.2):
 
 
 def time_moe(hip, ctx, steps, warmup, seed, mode, settle_s=0.2, dtype=None):
-    """configs[3]: 8 Q4_0 experts (w1 14336x4096, w2 4096x14336), 256 tokens,
+    """8 Q4_0 experts (w1 14336x4096, w2 4096x14336), 256 tokens,
     top-2 of N(0,1) router logits; ms per grouped-FFN call (all 8 experts'
     weights stream from HBM each call), the touched weight bytes, and a
     sample of the first 8 tokens (checked in the CPU leg).  dtype: the same
@@ -295,7 +295,7 @@ LLAMA_WEIGHT_BYTES = 598_757_376  # 22 x 24,772,608 B of Q4_K linears + the 53,7
 
 
 def llama_weights(seed):
-    """configs[4]: TinyLlama-shaped random decoder, every weight N(0, 0.02)
+    """TinyLlama-shaped random decoder, every weight N(0, 0.02)
     quantized (Q4_K linears and token_embd, Q6_K head), norms = 1."""
     import rce_amd
     G = rce_amd.GgufDtype
@@ -626,7 +626,7 @@ def main():
     mode = Mode.Q8 if args.mode == "q8" else Mode.EXACT
     rows = set() if args.quick else set(r for r in args.rows.split(",") if r)
 
-    # ---- headline: configs[1], Q4_0 11008x4096, batch 1 -------------------------
+    # ---- headline: Q4_0 11008x4096, batch 1 -------------------------
     dt, n, k = G.Q4_0, 11008, 4096
     log(f"headline Q4_0 GEMV {n}x{k} batch 1 mode={args.mode} steps={args.steps} warmup={args.warmup}")
     ms, b, x, res, copies = time_gemv(hip, ctx, dt, n, k, 1, mode, args.steps, args.warmup, 11, settle_s=0.3)
@@ -657,7 +657,7 @@ def main():
         "dtype": "int8" if mode == Mode.Q8 else "f32",
         "data": "synthetic: W~N(0,0.02) seeded then GGUF-quantized, x~N(0,1); weights rotated over "
                 f"{copies} HBM copies",
-        "config": {"workload": "configs[1]: Q4_0 GEMV 11008x4096 batch 1", "mode": args.mode,
+        "config": {"workload": "Q4_0 GEMV 11008x4096 batch 1", "mode": args.mode,
                    "bytes_per_launch": nbytes},
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4),
@@ -671,14 +671,14 @@ def main():
     kept = {}
     if "sweep" in rows:
         sweep = [
-            ("Q8_0 4096x4096 b1", G.Q8_0, 4096, 4096, 1),      # configs[0] shape
-            ("Q4_0 11008x4096 b1", G.Q4_0, 11008, 4096, 1),    # configs[1]
-            ("Q4_0 11008x4096 b8", G.Q4_0, 11008, 4096, 8),    # configs[1], batch 8
+            ("Q8_0 4096x4096 b1", G.Q8_0, 4096, 4096, 1),
+            ("Q4_0 11008x4096 b1", G.Q4_0, 11008, 4096, 1),
+            ("Q4_0 11008x4096 b8", G.Q4_0, 11008, 4096, 8),
             ("Q4_K 4096x4096 b1", G.Q4K, 4096, 4096, 1),
-            ("Q4_K 5632x2048 b1", G.Q4K, 5632, 2048, 1),       # configs[4] FFN shapes
+            ("Q4_K 5632x2048 b1", G.Q4K, 5632, 2048, 1),       # the decoder's FFN shapes
             ("Q4_K 2048x5632 b1", G.Q4K, 2048, 5632, 1),
             ("Q5_K 4096x4096 b1", G.Q5K, 4096, 4096, 1),       # Q5_K_M models' linears
-            ("Q6_K 32000x2048 b1", G.Q6K, 32000, 2048, 1),     # configs[4] head
+            ("Q6_K 32000x2048 b1", G.Q6K, 32000, 2048, 1),     # the decoder's head
             ("Q5_0 4096x4096 b1", G.Q5_0, 4096, 4096, 1),
             ("Q4_1 4096x4096 b1", G.Q4_1, 4096, 4096, 1),
             ("Q3_K 4096x4096 b1", G.Q3K, 4096, 4096, 1),
@@ -699,7 +699,7 @@ def main():
                 key = f"{name} {m.name.lower()}"
                 per[key] = {"us": round(sms * 1e3, 2), "GB/s": round(sg, 1), "hbm_frac": round(sg / HBM_PEAK_GBS, 4)}
                 log(f"  {key}: {sms * 1e3:.2f} us  {sg:.0f} GB/s ({sg / HBM_PEAK_GBS:.1%})")
-    if "gemm" in rows:  # configs[2]: Q4_K prefill GEMM 512x4096x4096 on f16 MFMA, then the other formats
+    if "gemm" in rows:  # Q4_K prefill GEMM 512x4096x4096 on f16 MFMA, then the other formats
         for gdt in (G.Q4K, G.Q6K, G.Q8_0, G.Q5K, G.Q5_0, G.Q4_1, G.BF16, G.F32):
             gms, gs = time_gemm(hip, ctx, gdt, 4096, 4096, 512, max(20, args.steps // 4), 5, 300)
             gtf = 2.0 * 512 * 4096 * 4096 / (gms * 1e-3) / 1e12
@@ -714,7 +714,7 @@ def main():
         key = "Q4_K GEMM 64x4096x4096 f16_mfma"
         per[key] = {"us": round(gms * 1e3, 2), "TFLOP/s": round(gtf, 1), "mfma_frac": round(gtf / MFMA_F16_PEAK_TFS, 4)}
         log(f"  {key}: {gms * 1e3:.2f} us  {gtf:.0f} TFLOP/s ({gtf / MFMA_F16_PEAK_TFS:.1%} of f16 MFMA peak)")
-    if "moe" in rows:  # configs[3]: grouped MoE, 8 Q4_0 experts, 256 tokens, top-2
+    if "moe" in rows:  # grouped MoE, 8 Q4_0 experts, 256 tokens, top-2
         mms, mbytes, msample = time_moe(hip, ctx, 5, 2, 400, Mode.F16_MFMA)
         mtf = 120259084288 / (mms * 1e-3) / 1e12
         mgb = mbytes / (mms * 1e-3) / 1e9
@@ -722,7 +722,7 @@ def main():
         per[key] = {"us": round(mms * 1e3, 2), "TFLOP/s": round(mtf, 1), "mfma_frac": round(mtf / MFMA_F16_PEAK_TFS, 4),
                     "GB/s": round(mgb, 1), "hbm_frac": round(mgb / HBM_PEAK_GBS, 4)}
         kept["moe"] = dict(msample, key=key)
-        log(f"  MoE configs[3]: {mms * 1e3:.1f} us  {mtf:.0f} TFLOP/s ({mtf / MFMA_F16_PEAK_TFS:.1%}), "
+        log(f"  MoE: {mms * 1e3:.1f} us  {mtf:.0f} TFLOP/s ({mtf / MFMA_F16_PEAK_TFS:.1%}), "
             f"{mgb:.0f} GB/s ({mgb / HBM_PEAK_GBS:.1%})")
         # the same workload with the expert formats Q4_K_M / Q5_K_M / Q8_0 models ship
         for mdt, mname in ((G.Q6K, "Q6_K"), (G.Q5K, "Q5_K"), (G.Q8_0, "Q8_0")):
@@ -736,8 +736,8 @@ def main():
             kept[f"moe {mname}"] = dict(msample, key=key)
             log(f"  {key}: {mms * 1e3:.1f} us  {mtf:.0f} TFLOP/s ({mtf / MFMA_F16_PEAK_TFS:.1%}), "
                 f"{mgb:.0f} GB/s ({mgb / HBM_PEAK_GBS:.1%})")
-    if "llama" in rows:  # configs[4]: TinyLlama-shaped decode, batch 1
-        log("  building the configs[4] decoder (22 layers, Q4_K + Q6_K head)")
+    if "llama" in rows:  # TinyLlama-shaped decode, batch 1
+        log("  building the TinyLlama-shaped decoder (22 layers, Q4_K + Q6_K head)")
         W = llama_weights(500)
         lsteps, lwarm = 128, 16
         # Q8, then the reference-order EXACT mode

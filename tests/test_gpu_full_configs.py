@@ -1,6 +1,6 @@
-"""GPU parity at the full workloads of configs[3] and configs[4].
+"""GPU parity at the full benchmark workloads of the decoder and the grouped experts.
 
-the TinyLlama-shaped decoder (22 layers, d 2048, ffn 5632, 32 q /
+The TinyLlama-shaped decoder (22 layers, d 2048, ffn 5632, 32 q /
 4 kv heads, d_head 64, Q4_K linears and token_embd, Q6_K 32000 x 2048 head,
 norms = 1, every weight N(0, 0.02) quantized by the reference's encoders),
 batch-1 decode over 72 positions, so attention runs past one 64-key run.
@@ -19,7 +19,7 @@ batch-1 decode over 72 positions, so attention runs past one 64-key run.
     1e-2 .. 5e-2 normwise at 22 layers); the test reports both and bounds
     the device's by the Q8 noise level, TOL_Q8_FULL.
 
-8 Q4_0 experts (w1 14336 x 4096, w2 4096 x 14336), 256 tokens
+Grouped experts: 8 Q4_0 experts (w1 14336 x 4096, w2 4096 x 14336), 256 tokens
 N(0, 1), top-2 of N(0, 1) router logits (rce-qwen36-moe/src/lib.rs L667-710,
 rce-op-moe L35-110).  The device runs all 256 tokens in each mode, and all
 256 are compared with the oracle:
@@ -56,8 +56,8 @@ def note(msg):
 
 @pytest.fixture(scope="module")
 def tl(ctx):
-    """The configs[4] weights on the host and, once, on the device."""
-    note("configs[4] weights: 22 layers, Q4_K linears, Q6_K head (quantizing)")
+    """The decoder's weights on the host and, once, on the device."""
+    note("decoder weights: 22 layers, Q4_K linears, Q6_K head (quantizing)")
     W = make_weights(TL_CFG, seed=500, sigma=0.02, unit_norms=True)
     sh = shapes(TL_CFG)
     qw = lambda bd, n, k: rce_amd.QuantWeight.from_owned_bytes(ctx, bd[0], bd[1], n, k)  # noqa: E731
@@ -97,7 +97,7 @@ def bits(x):
 
 def test_tinyllama_22_layers_exact(ctx, tl):
     W, dev, toks = tl
-    note(f"configs[4] EXACT, 22 layers, {N_POS} positions")
+    note(f"decoder EXACT, 22 layers, {N_POS} positions")
     d = device_decoder(ctx, W, dev, Mode.EXACT, range(22))
     ref = oracle_decoder(W, False, range(22))
     same = oracle_decoder(W, False, range(22), device_order=(256, -256))  # fused layer norms, separate head norm
@@ -113,7 +113,7 @@ def test_tinyllama_22_layers_exact(ctx, tl):
 
 def test_tinyllama_22_layers_q8(ctx, tl):
     W, dev, toks = tl
-    note(f"configs[4] Q8, 22 layers, {N_POS} positions")
+    note(f"decoder Q8, 22 layers, {N_POS} positions")
     d = device_decoder(ctx, W, dev, Mode.Q8, range(22))
     same = oracle_decoder(W, True, range(22), device_order=(256, 256))  # every norm fused
     ref = oracle_decoder(W, True, range(22))
@@ -132,14 +132,14 @@ def test_tinyllama_22_layers_q8(ctx, tl):
     assert max(dev_err) < TOL_Q8_FULL
 
 
-# ---- configs[3]: grouped experts ---------------------------------------------
+# ---- grouped experts ---------------------------------------------
 
 MOE_E, MOE_DM, MOE_DFF, MOE_T, MOE_K = 8, 4096, 14336, 256, 2
 
 
 @pytest.fixture(scope="module")
 def moe(ctx):
-    note("configs[3] experts: 8 x (14336x4096, 4096x14336) Q4_0 (quantizing)")
+    note("grouped experts: 8 x (14336x4096, 4096x14336) Q4_0 (quantizing)")
     rng = np.random.default_rng(400)
     q = lambda n, k: rce_amd.quantize(rng.standard_normal((n, k), dtype=F32) * F32(0.02), O.Q4_0)  # noqa: E731
     w1b = [q(MOE_DFF, MOE_DM) for _ in range(MOE_E)]
@@ -182,7 +182,7 @@ def moe_ref(moe):
 
 def test_moe_full_f16_mfma(ctx, moe, moe_ref):
     _, _, x, ids, gw, W1, W2, sample = moe
-    note("configs[3] F16_MFMA, 8 experts x 256 tokens top-2")
+    note("grouped experts F16_MFMA, 8 experts x 256 tokens top-2")
     got = run_full_moe(ctx, W1, W2, x, ids, gw, Mode.F16_MFMA)
     err = normwise(got[sample], moe_ref)
     note(f"  normwise {err:.3e} over all tokens")
@@ -191,7 +191,7 @@ def test_moe_full_f16_mfma(ctx, moe, moe_ref):
 
 def test_moe_full_exact(ctx, moe, moe_ref):
     w1b, w2b, x, ids, gw, W1, W2, sample = moe
-    note("configs[3] EXACT, 8 experts x 256 tokens top-2")
+    note("grouped experts EXACT, 8 experts x 256 tokens top-2")
     got = run_full_moe(ctx, W1, W2, x, ids, gw, Mode.EXACT)
     err = normwise(got[sample], moe_ref)
     note(f"  normwise {err:.3e} over all tokens")
@@ -202,7 +202,7 @@ def test_moe_full_exact(ctx, moe, moe_ref):
 
 def test_moe_full_q8(ctx, moe):
     w1b, w2b, x, ids, gw, W1, W2, sample = moe
-    note("configs[3] Q8, 8 experts x 256 tokens top-2")
+    note("grouped experts Q8, 8 experts x 256 tokens top-2")
     got = run_full_moe(ctx, W1, W2, x, ids, gw, Mode.Q8)
     same = O.moe_ffn(x[sample], w1b, w2b, O.Q4_0, MOE_DFF, ids[sample], gw[sample], q8=True, silu_dev=True)
     assert np.array_equal(got[sample].view(np.uint32), same.view(np.uint32))

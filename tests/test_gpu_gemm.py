@@ -105,7 +105,7 @@ def normwise(got, want):
 
 
 CASES = [
-    # (dtype, n_rows, n_cols, tokens): the configs[2] shape, ragged M and N,
+    # (dtype, n_rows, n_cols, tokens): 512 x 4096 x 4096, ragged M and N,
     # short K (split-K off), Q4_0 (the MoE experts' format)
     (O.Q4_K, 4096, 4096, 512),
     (O.Q4_K, 384, 1024, 100),
@@ -175,7 +175,7 @@ def gen_weight_bytes(rng, dt, n, k):
 
 
 GEN_CASES = [
-    # (dtype, n_rows, n_cols, tokens): configs[2]'s shape for the three
+    # (dtype, n_rows, n_cols, tokens): 512 x 4096 x 4096 for the three
     # formats a Q4_K_M / Q5_K model's prefill needs besides Q4_K, then
     # ragged M and N (partial tiles, N not a multiple of the 64-row IL64
     # groups), chunk counts that are not multiples of the 6-deep load ring
@@ -197,7 +197,7 @@ GEN_CASES = [
     (O.Q8_0, 128, 448, 40),
     (O.F16, 96, 832, 20),
     (O.Q4_1, 64, 1600, 9),
-    # the bf16 forms (BF16 exact; F32 as two bf16 terms), configs[2]'s
+    # the bf16 forms (BF16 exact; F32 as two bf16 terms), the 512 x 4096 x 4096
     # shape and ragged ones
     (O.BF16, 4096, 4096, 512),
     (O.F32, 4096, 4096, 512),

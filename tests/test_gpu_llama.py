@@ -188,7 +188,7 @@ def test_llama_head_dim_128_runs_past_one_per_wave(ctx):
 
 @pytest.mark.parametrize("mode,tol", [(Mode.EXACT, 1e-5), (Mode.Q8, 1e-1)])
 def test_llama_tinyllama_width_long_context(ctx, mode, tol):
-    """configs[4] widths (d 2048, 32 q / 4 kv heads, d_head 64, ffn 5632, Q4_K
+    """The benchmark decoder's widths (d 2048, 32 q / 4 kv heads, d_head 64, ffn 5632, Q4_K
     linears, Q6_K 32000-row head) on 2 layers over 300 positions: from
     position 256 on, wave 0 merges its second 64-key run (run 4) into its
     first, with a finite running max.  Bit-identical to the
@@ -280,7 +280,7 @@ def test_llama_dev_entry_matches_host_entry(ctx):
 
 
 def test_llama_tinyllama_shape(ctx):
-    """configs[4] widths: d 2048, ffn 5632, 32 q / 4 kv heads, d_head 64,
+    """The benchmark decoder's widths: d 2048, ffn 5632, 32 q / 4 kv heads, d_head 64,
     Q4_K linears, Q6_K 32000 x 2048 head (2 of the 22 layers)."""
     note("llama TinyLlama shape, 2 layers")
     c = dict(d_model=2048, vocab=32000, n_layers=2, n_q_heads=32, n_kv_heads=4, d_head=64, rope_dim=64,

@@ -115,7 +115,7 @@ def test_moe_f16_mfma(ctx, E, dm, dff, t, k, dt):
 
 
 def test_moe_mixtral_shapes(ctx):
-    """configs[3] expert shapes (w1 14336x4096, w2 4096x14336, Q4_0) on two
+    """The benchmark's expert shapes (w1 14336x4096, w2 4096x14336, Q4_0) on two
     experts and a few tokens: the full-size tiles and long K of both GEMMs."""
     E, dm, dff, t, k, dt = 2, 4096, 14336, 6, 2, O.Q4_0
     note(f"moe mixtral-shaped E={E} t={t}")

@@ -79,7 +79,7 @@ def test_prior_is_on_the_reference_scale():
 @pytest.mark.parametrize("dt,n,k,want", [
     (G.Q8_0, 64, 64, "cpu:op-qmm"),          # tiny: the per-call overhead decides
     (G.Q4_0, 512, 1024, "cpu:op-qmm"),
-    (G.Q4_0, 11008, 4096, "hip:op-qmm"),     # configs[1]
+    (G.Q4_0, 11008, 4096, "hip:op-qmm"),
     (G.Q4K, 4096, 4096, "hip:op-qmm"),
     (G.Q3K, 2048, 2048, "hip:op-qmm"),
     (G.F16, 4096, 4096, "cpu:op-qmm"),       # no adapter id for F16: declined
