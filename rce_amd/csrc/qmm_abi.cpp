@@ -586,25 +586,26 @@ bool moe_q8_mfma_preferred(double rows_per_expert, bool q6, bool by_tile) {
 
 // EXACT grouped experts: all in one launch over tiles of one and two slots, or
 // one product per expert, which waits for the grouping on the host and makes
-// launches for every expert but, with many slots, uses the decode kernels'
-// shapes of up to 16 rows per lane.  `m` is the multiply-adds of the call in 10^6.  Fitted
-// to 4 and 8 experts top-1 and top-2 of 1024x2816, 2048x5632 and 4096x14336 at 16-256 tokens: the
-// launches and the wait cost 40 us and 10 per expert; the tiles cost more per
-// 10^6 by 0.018 us (Q8_0, Q4_1, Q5_K), 0.010 (Q4_K), 0.007 (Q4_0, Q5_0, Q3_K), nothing (Q6_K, one
-// kernel for both).  One product per expert / tiles (us), 8 experts top-2, 2048x5632 at 64
-// and 256 tokens: Q8_0 460 / 373, 1241 / 1361; Q5_K 1426 / 1527 at 256; Q4_0 518 / 371, 1428 /
-// 1327; 4096x14336 at 16, 64 and 256: Q8_0 595 / 544, 1721 / 1764, 6126 / 6821; Q4_0 634 / 487, 1685 /
-// 1597, 5917 / 6194; Q6_K 20542 / 20421 at 256.
-bool moe_exact_tiles_preferred(uint32_t t1, uint32_t t2, size_t n_expert, double m1, double m2) {
-    auto extra = [](uint32_t t) {
-        switch (t) {
-        case T_Q6_K: return 0.0;
-        case T_Q4_0: case T_Q5_0: case T_Q3_K: return 0.007;
-        case T_Q4_K: return 0.010;
-        default: return 0.018;
+// launches for every expert.  m1, m2: the multiply-adds of the call with either matrix in 10^6.
+// The launches and the wait cost 40 us and 10 per expert; the tiles cost more only
+// in rows of more than 256 units of 32 values (K > 8192), per 10^6 0.017 us (Q8_0, Q4_1)
+// or 0.011.  Fitted to seven formats, 4-32 experts top-2 of 1024x2816 to 8192x8192,
+// 2048x14336, 14336x2048 and 4096x14336 at 4-256 tokens, routed at random and all
+// to two experts (670 calls): the form taken is within 3 % of the faster one at all of them.  One
+// product per expert / tiles (us), 8 experts, 256 tokens at random and all to two
+// experts: 2048x5632 Q8_0 1241 / 1116, 1133 / 1102, Q4_0 1411 / 1258, 1299 /
+// 1246; 4096x14336 Q8_0 6073 / 6500, 5973 / 6492, Q4_0 5871 / 6018, 5743 / 5979, Q5_K 5940 / 5796,
+// 5719 / 5782; 64 tokens Q8_0 1614 / 1628, Q4_0 1671 / 1533.
+bool moe_exact_tiles_preferred(const DevWeight &w1, const DevWeight &w2, size_t n_expert, double m1, double m2) {
+    auto extra = [](const DevWeight &w) {
+        if (w.n_cols <= 8192) return 0.0;
+        switch (w.dtype) {
+        case T_Q8_0: case T_Q4_1: return 0.017;
+        case T_Q4_0: case T_Q5_0: case T_Q3_K: return 0.011;
+        default: return 0.0;
         }
     };
-    return extra(t1) * m1 + extra(t2) * m2 < 40.0 + 10.0 * (double)n_expert;
+    return extra(w1) * m1 + extra(w2) * m2 < 40.0 + 10.0 * (double)n_expert;
 }
 
 // The grouped experts: h = silu(W1 x) (w3 == nullptr, the benchmark's
@@ -671,7 +672,7 @@ rce_qmm_status moe_run(rce_qmm_context *ctx, const rce_qmm_weight *const *w1, co
         if (args && gemv_grouped_supports(a1.dtype, d_model, (int)mode) && gemv_grouped_supports(a2.dtype, d_ff, (int)mode))
             form = BY_TILE;
         const double m = (double)n_pairs * (double)d_model * (double)d_ff * 1e-6;
-        if (mode == RCE_QMM_MODE_EXACT && !moe_exact_tiles_preferred(a1.dtype, a2.dtype, n_expert, w3 ? 2.0 * m : m, m)) form = BY_EXPERT;
+        if (mode == RCE_QMM_MODE_EXACT && !moe_exact_tiles_preferred(a1, a2, n_expert, w3 ? 2.0 * m : m, m)) form = BY_EXPERT;
         const size_t tiles16 = n_pairs / 16 + n_expert;
         if (args && mode == RCE_QMM_MODE_Q8 && gemv_q8_grouped_supports(a1, tiles16) && gemv_q8_grouped_supports(a2, tiles16) &&
             moe_q8_mfma_preferred(per_expert, a1.dtype == T_Q6_K || a2.dtype == T_Q6_K, form != BY_EXPERT))

@@ -1612,7 +1612,11 @@ hipError_t launch_as_preq_tb(const DevWeight &w, const GemvGeom &g, const float 
 
 // Grouped experts (FX_GROUP): one or two slots per block; the most rows per
 // lane (8, 4, 2) whose addends fit the LDS and that leave two blocks per CU
-// when every tile is present.
+// when every tile is present.  EXACT with two slots: 16 where that leaves
+// three blocks per CU, as several tokens of the plain product take (both
+// matrices at 16 against 8: 2048x5632 with 8 experts, 128 tokens top-2, Q4_1 570 /
+// 448 us, Q8_0 711 / 615; from 768 blocks on 0.78-1.01 of the time but for one
+// call of 402, at 512-768 up to 1.05).
 template <class Unit, int NT, int RPL, bool Q8>
 hipError_t launch_as_grouped(const DevWeight &w, int U, const MoeGroup &m, const void *a, float *out, hipStream_t s) {
     constexpr int TB = Unit::NTOK;
@@ -1639,10 +1643,13 @@ hipError_t launch_as_grouped(const DevWeight &w, int U, const MoeGroup &m, const
 template <class Unit, bool Q8>
 hipError_t launch_as_grouped_nt(const DevWeight &w, const MoeGroup &m, const void *a, float *out, hipStream_t s) {
     const int U = units_per_row(w.dtype, w.n_cols), nt = nt_for(U);
-    int rpl = 8;
+    constexpr bool TALL = !Q8 && Unit::NTOK == 2;
+    int rpl = TALL ? 16 : 8;
     auto blocks = [&](int r) { return (w.n_rows + (size_t)(nt / U) * r - 1) / ((size_t)(nt / U) * r) * (size_t)m.max_tiles; };
-    while (rpl > 2 && (gemv_lds_bytes(U, nt, rpl, Unit::NTOK, false, w.n_cols) > LDS_MAX || blocks(rpl) < 512)) rpl /= 2;
+    while (rpl > 2 && (gemv_lds_bytes(U, nt, rpl, Unit::NTOK, false, w.n_cols) > LDS_MAX || blocks(rpl) < (rpl == 16 ? 768 : 512))) rpl /= 2;
 #define RCE_GRP(NT)                                                              \
+    if constexpr (TALL)                                                          \
+        if (rpl == 16) return launch_as_grouped<Unit, NT, 16, Q8>(w, U, m, a, out, s); \
     switch (rpl) {                                                               \
     case 8: return launch_as_grouped<Unit, NT, 8, Q8>(w, U, m, a, out, s);       \
     case 4: return launch_as_grouped<Unit, NT, 4, Q8>(w, U, m, a, out, s);       \

@@ -115,17 +115,26 @@ def test_many_experts_expert_by_expert_q8(ctx, monkeypatch, mma):
     assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q4_0, dff, ids, gw, q8=True, silu_dev=True))
 
 
-@pytest.mark.parametrize("t", [1300, 1340])
-def test_exact_forms_on_both_sides_of_the_rule(ctx, t):
-    """One Q8_0 expert of 512 x 2048: 2726 and 2810 million multiply-adds, in tiles
-    of two slots and as a product of its own."""
-    print(f"moe exact rule t={t}", flush=True)
+@pytest.mark.parametrize("dm,dff,t", [(512, 2048, 1300), (512, 2048, 1340), (256, 8448, 1340), (256, 8448, 1380)])
+def test_exact_forms_on_both_sides_of_the_rule(ctx, dm, dff, t):
+    """One Q8_0 expert: short rows, in tiles of two slots at any size, and rows
+    of 264 blocks, 2898 and 2985 million multiply-adds, in tiles and as a
+    product of its own."""
+    print(f"moe exact rule d={dm} ff={dff} t={t}", flush=True)
     rng = np.random.default_rng(t)
-    w1, w2 = experts(rng, O.Q8_0, 1, 2048, 512), experts(rng, O.Q8_0, 1, 512, 2048)
-    x = rng.standard_normal((t, 512)).astype(np.float32)
+    w1, w2 = experts(rng, O.Q8_0, 1, dff, dm), experts(rng, O.Q8_0, 1, dm, dff)
+    x = rng.standard_normal((t, dm)).astype(np.float32)
     ids, gw = np.zeros((t, 1), np.int32), np.ones((t, 1), np.float32)
-    got = run_moe(ctx, w1, w2, O.Q8_0, 512, 2048, x, ids, gw, Mode.EXACT)
-    assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q8_0, 2048, ids, gw, silu_dev=True))
+    got = run_moe(ctx, w1, w2, O.Q8_0, dm, dff, x, ids, gw, Mode.EXACT)
+    assert bit_equal(got, O.moe_ffn(x, w1, w2, O.Q8_0, dff, ids, gw, silu_dev=True))
+
+
+@pytest.mark.parametrize("dt", [O.Q4_0, O.Q8_0, O.Q5_0, O.Q4_1, O.Q3_K, O.Q4_K, O.Q5_K])
+@pytest.mark.parametrize("t", [34, 41])
+def test_exact_sixteen_rows_per_lane(ctx, dt, t):
+    """Both matrices at 16 rows per lane (at least 768 blocks; at 34 tokens
+    the K-quants' first at 8), the last block of W2's rows part filled."""
+    check(ctx, dt, 4, 4096, 1280, t, 2, Mode.EXACT)
 
 
 @pytest.mark.parametrize("mode", [Mode.EXACT, Mode.Q8])
